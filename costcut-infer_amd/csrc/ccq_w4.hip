@@ -29,6 +29,7 @@
 // layout.
 #include "ccq_common.h"
 #include "ccq_topk.h"
+#include "ccq_w4_mfma.h"
 
 #include <math.h>
 
@@ -45,10 +46,6 @@ __device__ __forceinline__ int tile_nib(int e) { return (e & 1) ? 4 + (e >> 1) :
 __device__ __forceinline__ float scale_at(const uint16_t* s, int64_t i, int bf16) {
   uint32_t b = s[i];
   return bf16 ? bf16_bits_to_f32(b) : f16_bits_to_f32(b);
-}
-
-__host__ __device__ inline int64_t sz_words_per_column(int64_t K, int64_t G) {
-  return ((K / 128 + 3) / 4) * 4 * (128 / G);
 }
 
 // ------------------------------------------------------------------ dequant --
@@ -122,73 +119,7 @@ __global__ void awq_pack_sz_kernel(const uint32_t* __restrict__ qz, const uint16
   }
 }
 
-// ------------------------------------------------------------- MFMA pieces --
-template <typename AT>
-struct Act;
-template <>
-struct Act<__bf16> {
-  using vec = bf16x8;
-  static constexpr uint32_t kMagic2 = 0x43004300u;  // bf16 128.0 twice
-  static constexpr float kMagic = 128.0f;
-  static constexpr uint32_t kOne2 = 0x3F803F80u;
-};
-template <>
-struct Act<_Float16> {
-  using vec = f16x8;
-  static constexpr uint32_t kMagic2 = 0x64006400u;  // fp16 1024.0 twice
-  static constexpr float kMagic = 1024.0f;
-  static constexpr uint32_t kOne2 = 0x3C003C00u;
-};
-
-__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-// 32x32x16: A lane l = row l & 31, B lane l = column l & 31, both with
-// k = 8*(l >> 5) + e; D register i of lane l = (row 8*(i/4) + 4*(l >> 5) + i%4,
-// column l & 31).
-__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-template <typename AT>
-__device__ __forceinline__ typename Act<AT>::vec dq_b(uint32_t w) {
-  u32x4 r;
-  r[0] = (w & 0x000F000Fu) | Act<AT>::kMagic2;
-  r[1] = ((w >> 4) & 0x000F000Fu) | Act<AT>::kMagic2;
-  r[2] = ((w >> 8) & 0x000F000Fu) | Act<AT>::kMagic2;
-  r[3] = ((w >> 12) & 0x000F000Fu) | Act<AT>::kMagic2;
-  return __builtin_bit_cast(typename Act<AT>::vec, r);
-}
-
-// dq_b with one v_and_or_b32 per weight pair: the mask and the magic come in
-// as run-time values (an SGPR and a VGPR), since a VOP3 op on gfx9 takes no
-// literal and (w & literal) | literal would cost two ops.
-template <typename AT>
-__device__ __forceinline__ typename Act<AT>::vec dq_b3(uint32_t w, uint32_t mask_s, uint32_t magic_v) {
-  u32x4 r;
-  r[0] = (w & mask_s) | magic_v;
-  r[1] = ((w >> 4) & mask_s) | magic_v;
-  r[2] = ((w >> 8) & mask_s) | magic_v;
-  r[3] = ((w >> 12) & mask_s) | magic_v;
-  return __builtin_bit_cast(typename Act<AT>::vec, r);
-}
-
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
-
-__device__ __forceinline__ void store_val(void* y, int64_t i, float v, int dt) {
-  if (dt == CCQ_F32)
-    reinterpret_cast<float*>(y)[i] = v;
-  else if (dt == CCQ_BF16)
-    reinterpret_cast<uint16_t*>(y)[i] = (uint16_t)f32_to_bf16_bits(v);
-  else
-    reinterpret_cast<uint16_t*>(y)[i] = (uint16_t)f32_to_f16_bits(v);
-}
 
 // ---------------------------------------------------------- skinny kernel --
 enum { EPI_STORE = 0, EPI_SILU = 1, EPI_ROWS = 2 };
@@ -218,17 +149,6 @@ struct SkinnyP {
 // k-tiles whose packed weights, scales and zeros one wave holds in registers
 // at once: all of them are requested before the first multiply.
 constexpr int KTW = 4;
-
-template <typename ST>
-__device__ __forceinline__ float sz_scale(uint32_t word);
-template <>
-__device__ __forceinline__ float sz_scale<__bf16>(uint32_t word) {
-  return __uint_as_float(word << 16);
-}
-template <>
-__device__ __forceinline__ float sz_scale<_Float16>(uint32_t word) {
-  return f16_bits_to_f32(word & 0xFFFFu);
-}
 
 // One workgroup job: the 16-row tile `tile` times the 16*NB output columns of
 // block `nb`, K split over the W waves (wave w owns k-tiles
@@ -1901,7 +1821,9 @@ bool gemm_grouped(int64_t M, int64_t K, int64_t N, int64_t G) {
 }  // namespace
 
 extern "C" size_t ccq_w4_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size) {
-  if (M <= 0 || K <= 0 || K % 128 || !gemm_grouped(M, K, N, group_size)) return 0;
+  if (M <= 0 || K <= 0 || K % 128 || N <= 0 || !valid_group(group_size)) return 0;
+  if (w4_slab_takes(M, K, N, group_size)) return w4_slab_workspace(M, K, N);
+  if (!gemm_grouped(M, K, N, group_size)) return 0;
   // row group sums, then the row ids of the 128-row tiles
   return align256((size_t)M * (size_t)(K / 128) * 4) + align256((size_t)cdiv(M, GG_BM) * GG_BM * 4);
 }
@@ -1985,6 +1907,11 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
     w.szw = (int)szw_d;
     w.nib_mask = 0x000F000Fu;
     return launch_stream<EPI_STORE>(w, nq, x_dtype == CCQ_BF16, scale_dtype == CCQ_BF16, 1, as_stream(stream));
+  }
+  if (w4_slab_takes(M, K, N, group_size)) {
+    const W4DenseP d = {x, (const uint32_t*)w_tiled, sz, y, x_dtype == CCQ_BF16, scale_dtype == CCQ_BF16, y_dtype,
+                        M, K, N, group_size};
+    return launch_w4_slab(d, workspace, workspace_bytes, as_stream(stream));
   }
   const int64_t tiles = cdiv(M, 16);
   const SkinnyPlan pl = plan_skinny(K, N, group_size, 1, gemm_nb(M));

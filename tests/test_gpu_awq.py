@@ -108,6 +108,38 @@ def test_gemm_parity_groups(gpu, G):
     assert _gemm_case(gpu, 3, 384, 160, G, torch.float16, torch.float32, seed=G) <= TIGHT
 
 
+@pytest.mark.parametrize("M,K,N,G", [(17, 4096, 9232, 128), (33, 4480, 6160, 128), (49, 1152, 11024, 128),
+                                     (64, 4224, 5200, 64), (40, 3200, 7184, 64), (32, 2176, 9232, 32),
+                                     (48, 4480, 5136, 32), (64, 3200, 4112, 32)])
+def test_gemm_slab_kernel(gpu, M, K, N, G):
+    """17 to 64 rows on enough columns that the 16-row kernel would need a
+    second round of workgroups: 2, 3 and 4 row tiles, part-filled last rows and
+    columns, k-tile counts that are no multiple of a step's, K split in two
+    (K=4480 with few columns) and without the workspace of a split."""
+    assert _gemm_case(gpu, M, K, N, G, torch.bfloat16, torch.float32, seed=M) <= TIGHT
+    assert _gemm_case(gpu, M, K, N, G, torch.float16, torch.float16, seed=M + 1) <= TOL
+
+
+def test_gemm_slab_kernel_without_workspace(gpu):
+    """A caller that passes no workspace gets the unsplit kernel, equal up to
+    the order of the float32 sums."""
+    from ccut import _dev
+    from ccut._lib import call, lib
+    from ccut.quant import awq
+
+    M, K, N, G = 33, 4480, 6160, 128
+    assert lib().ccq_w4_gemm_workspace_size(M, K, N, G) == 2 * M * N * 4
+    qw, qz, s = _make(K, N, G, 7)
+    w = awq.prepare(torch.from_numpy(qw).to(gpu), torch.from_numpy(qz).to(gpu), torch.from_numpy(s).to(gpu), G)
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(7)).to(torch.bfloat16).to(gpu)
+    y = torch.empty((M, N), dtype=torch.float32, device=gpu)
+    call("ccq_w4_gemm", x.data_ptr(), 2, w.w_tiled.data_ptr(), w.sz.data_ptr(), 1, y.data_ptr(), 0, M, K, N, G, None, 0,
+         _dev.stream_ptr())
+    ref = awq.gemm(x, w, out_dtype=torch.float32)
+    # each is within K * 2^-24 of the exact sum of terms up to (MAGIC + 15) / 15 times its own
+    assert (y - ref).abs().max() <= TIGHT * ref.abs().max()
+
+
 def test_gemm_config_single_linear_k2048_n5632(gpu):
     """x fp16 [1, 2048], W int4 2048 -> 5632, group 128, fp16 out."""
     err = _gemm_case(gpu, 1, 2048, 5632, 128, torch.float16, torch.float16, seed=1)
