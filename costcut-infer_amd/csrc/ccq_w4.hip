@@ -1216,6 +1216,7 @@ struct W4GP {
   int64_t ldsxo;
   int M, N, K, KT, szw;
   uint32_t nib_mask;           // 0x000F000F (a run-time value, see dq_b3)
+  int splits;                  // EPI_STORE: K splits, float32 partials at y + split * M * N (1 = none)
 };
 
 constexpr int GG_BM = 128;
@@ -1261,7 +1262,17 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   // an XCD, workgroup wx takes every nx-th of the XCD's items (tile-major).
   const int xcd = blockIdx.x & 7, wx = blockIdx.x >> 3;
   const int nx = ((int)gridDim.x - xcd + 7) >> 3;
-  const int items_x = (ntiles > xcd ? (ntiles - xcd + 7) >> 3 : 0) * nblk;
+  // A dense weight (EPI_STORE) has as many row tiles as M / 128, often fewer
+  // than XCDs, so its items are dealt to the XCDs in contiguous ranges of the
+  // order (split, column block, row tile), as many items as the XCD's share of
+  // the grid: a column block's weights are read into one L2.  (Row tiles dealt
+  // round-robin left a single tile on one XCD: M=128 K=4096 N=14336 531 us;
+  // column blocks innermost, M=2048 305 us against 292.)
+  constexpr bool DENSE = EPI == EPI_STORE;
+  const int all = ntiles * nblk * (DENSE ? p.splits : 1);
+  const int first = DENSE ? xcd * (all >> 3) + min(xcd, all & 7) : 0;
+  const int items_x = DENSE ? (all >> 3) + (xcd < (all & 7) ? 1 : 0)
+                            : (ntiles > xcd ? (ntiles - xcd + 7) >> 3 : 0) * nblk;
   if (wx >= items_x) return;
   // Items are dealt in rounds of nx, alternating direction: the workgroup
   // that takes a round's first item takes the next round's last.  The
@@ -1271,12 +1282,18 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   // round-robin: T=512 top-8 layer, 128 experts, gate/up -5%, down -13%).
   auto item_of = [&](int j) { return j * nx + ((j & 1) ? nx - 1 - wx : wx); };
   const int nmine = items_x / nx + (item_of(items_x / nx) < items_x ? 1 : 0);
-  const int KT = p.KT;
+  const int per = DENSE ? ntiles * nblk : 1;  // items of one split
+  // a split K (then one item per workgroup, see launch_group_gemm) starts at kt0
+  const int split0 = DENSE && p.splits > 1 ? (first + item_of(0)) / per : 0;
+  const int kt0 = DENSE ? (int)((int64_t)p.KT * split0 / p.splits) : 0;
+  const int KT = DENSE ? (int)((int64_t)p.KT * (split0 + 1) / p.splits) - kt0 : p.KT;
   const int total = nmine * KT;  // k-steps of this workgroup
 
   // ---- row ids: rows of item j go to Rid[j % 3], copied (DMA) at the first
   // k-step of item j - 2; Rid[.][GG_BM..] holds the item's expert ----
-  auto tile_of = [&](int j) { return xcd + 8 * (item_of(j) / nblk); };
+  auto tile_of = [&](int j) {
+    return DENSE ? (first + item_of(j)) % per % ntiles : xcd + 8 * (item_of(j) / nblk);
+  };
   auto fetch_rows = [&](int j) {  // waves 5..7
     if (j >= nmine) return;
     const int tile = tile_of(j);
@@ -1304,7 +1321,7 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   const bool has_sx = wave == 4 || wave == 5;
   const int ncopy = 4 + BPW + (has_sz ? 1 : 0) + (has_sx ? 1 : 0);
   auto make_plan = [&](int j, Plan& P) {
-    P.nb = item_of(j) % nblk;
+    P.nb = DENSE ? (first + item_of(j)) % per / ntiles : item_of(j) % nblk;
     const int* R = Rid[j % 3];
     const int ex = p.tile_expert != nullptr ? __builtin_amdgcn_readfirstlane(R[GG_BM]) : 0;
     // valid rows form a prefix of the tile
@@ -1322,7 +1339,7 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
 #pragma unroll
     for (int b2 = 0; b2 < BPW; ++b2) {
       const int b = wave * BPW + b2, q = b / TPM, nt = P.nb * TPM + (b - q * TPM);
-      P.bsrc[b2] = reinterpret_cast<const char*>((q == 0 ? p.w0 : p.w1) + (int64_t)ex * p.w_es + (int64_t)nt * KT * 256);
+      P.bsrc[b2] = reinterpret_cast<const char*>((q == 0 ? p.w0 : p.w1) + (int64_t)ex * p.w_es + (int64_t)nt * p.KT * 256);
     }
     P.zsrc = nullptr;
     P.zoff = 0;
@@ -1341,6 +1358,7 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   const uint32_t lds0 = lds_addr(smem);
   auto issue = [&](const Plan& P, int kt, int slot) {
     const uint32_t st = lds0 + slot * GG_STAGE;
+    if constexpr (DENSE) kt += kt0;
     const char* xb = reinterpret_cast<const char*>(p.x) + (int64_t)kt * 256;
 #pragma unroll
     for (int i = 0; i < 4; ++i) dma16(xb, P.aoff[i], st + (16 * wave + 4 * i) * 256);
@@ -1546,7 +1564,7 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
             const float fr = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(fs), 0xB1, 0xF, 0xF, false));
             const float lo = odd ? fr : v0, hi = odd ? v1 : fr;  // columns (c & ~1), (c | 1) of the row
             if (row < P.nvalid) {
-              const int64_t o = (int64_t)R[row] * p.ldy + col2 + c * 32;
+              const int64_t o = (int64_t)R[row] * p.ldy + col2 + c * 32 + (DENSE ? (int64_t)split0 * p.M * p.N : 0);
               if (p.y_dtype == CCQ_F32)
                 *reinterpret_cast<f32x2*>(reinterpret_cast<float*>(p.y) + o) = f32x2{lo, hi};
               else if (p.y_dtype == CCQ_BF16)
@@ -1713,8 +1731,9 @@ static int launch_stream(const W4SP& p, int nq, int x_bf16, int s_bf16, int64_t 
 template <int EPI>
 static int launch_group_gemm(const W4GP& p, int x_bf16, int s_bf16, int64_t tiles, hipStream_t st) {
   const int wgn = group_cols(EPI, p.N);
-  const int64_t items = tiles * (p.N / wgn), cus = device_cus();
-  const dim3 grid((unsigned)(items < cus ? items : cus)), block(512);
+  const int64_t items = tiles * (p.N / wgn) * (EPI == EPI_STORE ? p.splits : 1), cus = device_cus();
+  // EPI_STORE deals items to all 8 XCDs: at least one workgroup each
+  const dim3 grid((unsigned)(EPI == EPI_STORE && items < 8 ? 8 : (items < cus ? items : cus))), block(512);
 #define CCQ_LAUNCH_GG(AT, ST)                                                                  \
   do {                                                                                         \
     if (wgn == 256)                                                                            \
@@ -1814,18 +1833,29 @@ extern "C" int ccq_awq_pack_sz(const int32_t* qzeros, const void* scales, int sc
 }
 
 namespace {
-// The dense GEMM switches to the grouped kernel for prefill-sized M.
-bool gemm_grouped(int64_t M, int64_t K, int64_t N, int64_t G) {
-  return M > 64 && G == 128 && N % 128 == 0 && K >= 256;
+// K splits of the grouped kernel: as many as give every CU an item of at least
+// 4 k-tiles.
+int group_splits(int64_t M, int64_t K, int64_t N) {
+  const int64_t items = cdiv(M, GG_BM) * (N / group_cols(EPI_STORE, N)), KT = K / 128;
+  int64_t s = device_cus() / items;
+  if (s > KT / 4) s = KT / 4;
+  return (int)(s < 1 ? 1 : s);
+}
+
+size_t group_partials(int64_t M, int64_t K, int64_t N) {
+  const int s = group_splits(M, K, N);
+  return s > 1 ? (size_t)s * (size_t)M * (size_t)N * 4 : 0;
 }
 }  // namespace
 
 extern "C" size_t ccq_w4_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size) {
   if (M <= 0 || K <= 0 || K % 128 || N <= 0 || !valid_group(group_size)) return 0;
   if (w4_slab_takes(M, K, N, group_size)) return w4_slab_workspace(M, K, N);
-  if (!gemm_grouped(M, K, N, group_size)) return 0;
+  if (!w4_grouped_takes(M, K, N, group_size)) return 0;
   // row group sums, then the row ids of the 128-row tiles
-  return align256((size_t)M * (size_t)(K / 128) * 4) + align256((size_t)cdiv(M, GG_BM) * GG_BM * 4);
+  // and the partial sums of a split K
+  return align256((size_t)M * (size_t)(K / 128) * 4) + align256((size_t)cdiv(M, GG_BM) * GG_BM * 4) +
+         group_partials(M, K, N);
 }
 
 extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, const uint32_t* sz, int scale_dtype,
@@ -1840,7 +1870,7 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
   CCQ_REQUIRE(y_dtype == CCQ_F16 || y_dtype == CCQ_BF16 || y_dtype == CCQ_F32, "ccq_w4_gemm: bad y_dtype");
   CCQ_REQUIRE(K <= (1 << 20) && N / 16 <= 0x7fffffff, "ccq_w4_gemm: K=%lld or N=%lld too large", (long long)K,
               (long long)N);
-  const bool grouped = gemm_grouped(M, K, N, group_size);
+  const bool grouped = w4_grouped_takes(M, K, N, group_size);
   CCQ_REQUIRE(grouped || cdiv(M, 16) <= 65535, "ccq_w4_gemm: M=%lld too large", (long long)M);
   if (M == 0 || N == 0) return 0;
   CCQ_REQUIRE(K > 0, "ccq_w4_gemm: K == 0");
@@ -1881,7 +1911,14 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
     g.KT = (int)(K / 128);
     g.szw = (int)sz_words_per_column(K, group_size);
     g.nib_mask = 0x000F000Fu;
-    return launch_group_gemm<EPI_STORE>(g, x_dtype == CCQ_BF16, scale_dtype == CCQ_BF16, g.tiles, st);
+    g.splits = group_splits(M, K, N);
+    if (g.splits > 1) {
+      g.y = (char*)rows + align256((size_t)tiles * GG_BM * 4);
+      g.y_dtype = CCQ_F32;
+    }
+    rc = launch_group_gemm<EPI_STORE>(g, x_dtype == CCQ_BF16, scale_dtype == CCQ_BF16, g.tiles, st);
+    if (rc || g.splits == 1) return rc;
+    return launch_w4_split_sum((const float*)g.y, y, y_dtype, g.splits, M * N, st);
   }
   const int64_t szw_d = sz_words_per_column(K, group_size);
   // 16-column jobs (one quad) when 32-column jobs would leave CUs idle

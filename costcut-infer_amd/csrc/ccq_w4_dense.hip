@@ -386,10 +386,17 @@ SlabPlan plan_slab(int64_t M, int64_t K, int64_t N) {
 // takes a second round and this kernel wins (M=33 K=4096 N=6144 17.9 against
 // 12.9, M=17 N=14336 22.5 against 13.9, M=37 34.3 against 17.6, M=64 46.7
 // against 24.1; G=32 M=64 67 against 32).
+//
+// Above 64 rows it takes, 64 rows at a time, what the 128-row grouped kernel
+// does not (group 32 or 64, N not a multiple of 128): G=64 K=4096 N=14336
+// M=128 86.9 -> 49.1 us, M=2048 1267 -> 671; G=32 M=2048 1963 -> 868.
+// Of the grouped kernel's shapes it takes those of one round of its blocks
+// (M=128 K=4096 N=4096 22.6 us of the 16-row kernel -> 16.4, M=130 K=7168
+// N=2432 34.5 -> 18.4; two rounds: M=65 K=2048 N=9216 15.1 against 20.2).
 bool w4_slab_takes(int64_t M, int64_t K, int64_t N, int64_t G) {
-  const int64_t waves = cdiv(M, 16) * cdiv(N, G == 32 ? 32 : 64) * imin64(8, cdiv(K / 128, 4));
-  return M > 16 && M <= 64 && waves > 256 * 8 && 64 * K * 2 < (1LL << 32) &&
-         N * sz_words_per_column(K, G) * 4 < (1LL << 32);
+  const int64_t blocks = cdiv(M, 64) * cdiv(N, 64);
+  return M > 16 && w4_skinny_waves(M, K, N, G) > 256 * 8 && (!w4_grouped_shape(M, K, N, G) || blocks <= 256) &&
+         64 * K * 2 < (1LL << 32) && N * sz_words_per_column(K, G) * 4 < (1LL << 32) && blocks <= 0x7fffffff;
 }
 
 size_t w4_slab_workspace(int64_t M, int64_t K, int64_t N) {
@@ -425,9 +432,11 @@ int launch_w4_slab(const W4DenseP& d, void* workspace, size_t workspace_bytes, h
     launch_slab_mt<_Float16>(p, pl.mt, ng, grid, st);
   int rc = launch_status("w4 slab gemm");
   if (rc || pl.splits == 1) return rc;
-  const int64_t n4 = d.M * d.N / 4;
-  launch(w4_split_sum_kernel, dim3((unsigned)cdiv(n4, 256)), dim3(256), 0, st, (const float*)workspace, d.y, d.y_dtype,
-         pl.splits, n4);
+  return launch_w4_split_sum((const float*)workspace, d.y, d.y_dtype, pl.splits, d.M * d.N, st);
+}
+
+int launch_w4_split_sum(const float* part, void* y, int y_dtype, int splits, int64_t n, hipStream_t st) {
+  launch(w4_split_sum_kernel, dim3((unsigned)cdiv(n / 4, 256)), dim3(256), 0, st, part, y, y_dtype, splits, n / 4);
   return launch_status("w4 split sum");
 }
 

@@ -98,8 +98,29 @@ struct W4DenseP {
   int x_bf16, s_bf16, y_dtype;
   int64_t M, K, N, G;
 };
+// Waves of the 16-row kernel's grid (w4_skinny_kernel): its weight passes times
+// its workgroups of up to 8 waves on 64 (G = 32: 32) columns.
+inline int64_t w4_skinny_waves(int64_t M, int64_t K, int64_t N, int64_t G) {
+  return cdiv(M, 16) * cdiv(N, G == 32 ? 32 : 64) * imin64(8, cdiv(K / 128, 4));
+}
+// Shapes of the 128-row grouped kernel.
+inline bool w4_grouped_shape(int64_t M, int64_t K, int64_t N, int64_t G) {
+  return M > 64 && G == 128 && N % 128 == 0 && K >= 256;
+}
+// It takes them unless the 16-row kernel does them in two rounds of the 256
+// CUs (8 waves each) or the slab kernel in one round of its 64 x 64 blocks:
+// the grouped kernel's row sums, split-K sums and launches cost about 20 us
+// by themselves (M=128 K=2048 N=2048 10.4 us against 22.0, M=65 K=2048 N=9216
+// 15.1 against 24, both the 16-row kernel; M=256 K=4096 N=4096 33 against 17
+// of the slab kernel; past those M=400 K=4096 N=4096 39 against 76 and M=128
+// K=4096 N=14336 40 against 81 and 50).
+inline bool w4_grouped_takes(int64_t M, int64_t K, int64_t N, int64_t G) {
+  return w4_grouped_shape(M, K, N, G) && w4_skinny_waves(M, K, N, G) > 2 * 256 * 8 && cdiv(M, 64) * cdiv(N, 64) > 256;
+}
 bool w4_slab_takes(int64_t M, int64_t K, int64_t N, int64_t G);
 size_t w4_slab_workspace(int64_t M, int64_t K, int64_t N);  // 0 when K is not split
+// y = the sum of `splits` float32 partials of n values each, n % 4 == 0
+int launch_w4_split_sum(const float* part, void* y, int y_dtype, int splits, int64_t n, hipStream_t st);
 int launch_w4_slab(const W4DenseP& p, void* workspace, size_t workspace_bytes, hipStream_t st);
 
 }  // namespace ccq

@@ -120,6 +120,24 @@ def test_gemm_slab_kernel(gpu, M, K, N, G):
     assert _gemm_case(gpu, M, K, N, G, torch.float16, torch.float16, seed=M + 1) <= TOL
 
 
+@pytest.mark.parametrize("M,K,N", [(65, 4096, 9216), (260, 3840, 3712), (257, 3712, 4352), (513, 1152, 2944),
+                                   (1150, 1152, 1152), (2100, 640, 2176)])
+def test_gemm_grouped_dense_schedule(gpu, M, K, N):
+    """The 128-row kernel on few and many row tiles: K split over 9, 10, 13 or
+    more workgroups per XCD share (odd k-tile counts, part-filled last tiles),
+    unsplit with several items per workgroup."""
+    assert _gemm_case(gpu, M, K, N, 128, torch.bfloat16, torch.float32, seed=M) <= TIGHT
+    assert _gemm_case(gpu, M, K, N, 128, torch.float16, torch.float16, seed=M + 1) <= TOL
+
+
+@pytest.mark.parametrize("M,K,N,G", [(65, 1152, 11024, 64), (129, 1024, 4096, 32), (200, 1152, 4112, 128),
+                                     (130, 7168, 2432, 128), (257, 3712, 2944, 128)])
+def test_gemm_slab_kernel_row_blocks(gpu, M, K, N, G):
+    """More than 64 rows: shapes the 128-row kernel does not take, and those of
+    its shapes whose 64 x 64 blocks are one round of the CUs."""
+    assert _gemm_case(gpu, M, K, N, G, torch.bfloat16, torch.float32, seed=M) <= TIGHT
+
+
 def test_gemm_slab_kernel_without_workspace(gpu):
     """A caller that passes no workspace gets the unsplit kernel, equal up to
     the order of the float32 sums."""
