@@ -31,7 +31,7 @@
 // barrier per chunk.  Weights (non-temporal loads), scale bytes and the
 // activation chunk are loaded PD chunks ahead into a register ring (PD 2-6,
 // wq_depth), so the wait for chunk c leaves chunks c+1..c+PD-1 in flight.
-#include "ccq_common.h"
+#include "ccq_wq.h"
 
 namespace ccq {
 
@@ -43,63 +43,6 @@ constexpr int WQ_THREADS = 512;            // 8 waves: 4 column groups x 2 k hal
 // as 8)
 constexpr int WQ_RS = WQ_KC + 8;
 constexpr int WQ_COLS = 16 * WQ_CG;        // output columns per workgroup
-
-struct WqP {
-  const float* x;
-  const uint8_t* w;
-  const void* scale;  // float [N] (row formats), E8M0 bytes [N, K / G] (MX), or null (MXFP4 only)
-  float* y;
-  int64_t M, K, N;
-  int G;
-  float s2;
-};
-
-template <int FMT>
-struct WqTraits {
-  static constexpr int WB = FMT == WQ_MXFP4 ? 1 : 2;      // 16-byte weight pieces per lane and chunk
-  static constexpr int KDIV = FMT == WQ_MXFP4 ? 2 : 1;    // k per weight byte
-  static constexpr bool MX = FMT == WQ_MXFP8 || FMT == WQ_MXFP4;
-};
-
-__device__ __forceinline__ bf16x8 pack_bf16x8(const float (&v)[8]) {
-  u32x4 r;
-  r[0] = bf16x2_bits(v[0], v[1]);
-  r[1] = bf16x2_bits(v[2], v[3]);
-  r[2] = bf16x2_bits(v[4], v[5]);
-  r[3] = bf16x2_bits(v[6], v[7]);
-  return __builtin_bit_cast(bf16x8, r);
-}
-
-// The lane's weight values 8i..8i+7 of the chunk (times the group scale s
-// for the MX formats) as the MFMA's B fragment.
-template <int FMT>
-__device__ __forceinline__ bf16x8 wq_decode(const u32x4 (&wr)[WqTraits<FMT>::WB], int i, float s) {
-  float v[8];
-  if constexpr (FMT == WQ_MXFP4) {
-    mx4_word(wr[0][i], v);
-  } else {
-    const uint32_t w0 = wr[i >> 1][(i & 1) * 2], w1 = wr[i >> 1][(i & 1) * 2 + 1];
-    if constexpr (FMT == WQ_INT8_ROW) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[j] = (float)(int8_t)(w0 >> (8 * j));
-        v[4 + j] = (float)(int8_t)(w1 >> (8 * j));
-      }
-    } else {
-      const auto a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w0, false);
-      const auto b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w0, true);
-      const auto c = __builtin_amdgcn_cvt_pk_f32_fp8((int)w1, false);
-      const auto d = __builtin_amdgcn_cvt_pk_f32_fp8((int)w1, true);
-      v[0] = a[0], v[1] = a[1], v[2] = b[0], v[3] = b[1];
-      v[4] = c[0], v[5] = c[1], v[6] = d[0], v[7] = d[1];
-    }
-  }
-  if constexpr (WqTraits<FMT>::MX) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] *= s;
-  }
-  return pack_bf16x8(v);
-}
 
 // Scale bytes of MXFP4 layers without scales: E8M0 127 (scale 1), read at
 // offset 0, so that every chunk issues the same loads.
@@ -297,7 +240,7 @@ int wq_mfma_linear(int fmt, const float* x, const uint8_t* w, const void* scale,
                    float* y, int64_t M, int64_t K, int64_t N, hipStream_t stream, const char* name) {
   const bool mx = fmt == WQ_MXFP8 || fmt == WQ_MXFP4;
   if (fmt < WQ_FP8_ROW || fmt > WQ_MXFP4) return -1;
-  if (M <= 0 || N <= 0 || K <= 0 || K % WQ_KC != 0) return -1;
+  if (M <= 0 || N <= 0 || K <= 0) return -1;
   if (!x || !w || !y || !aligned(x, 16) || !aligned(w, 16)) return -1;
   if (!mx && !scale) return -1;
   if (fmt == WQ_MXFP8 && !scale) return -1;
@@ -306,6 +249,9 @@ int wq_mfma_linear(int fmt, const float* x, const uint8_t* w, const void* scale,
   const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
   const WqP p{x, w, scale, y, M, K, N, mx && scale ? group_size : 32, scale2};
   const bool g16 = mx && scale && group_size == 16;
+  const int rc = wq_tile_linear(fmt, p, g16, stream, name);
+  if (rc >= 0) return rc;
+  if (K % WQ_KC != 0) return -1;
   switch (fmt) {
     case WQ_FP8_ROW: wq_launch<WQ_FP8_ROW, false>(mt, p, stream); break;
     case WQ_INT8_ROW: wq_launch<WQ_INT8_ROW, false>(mt, p, stream); break;

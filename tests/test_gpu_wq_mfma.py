@@ -147,3 +147,60 @@ def test_dispatch_through_layer_entries(gpu, batch):
         assert np.array_equal(y.cpu().numpy(), direct), entry
         ref = x.astype(np.float64) @ w.astype(np.float64).T
         assert np.max(np.abs(direct - ref)) <= 1e-5 * np.max(np.abs(ref))
+
+
+def _apply(gpu, fmt, x, raw, sc, s2, N, G):
+    """The layer entry point of the format (any in_features)."""
+    from ccut import _dev
+    from ccut._lib import call
+
+    M, K = x.shape
+    xd, rd = torch.from_numpy(x).to(gpu), torch.from_numpy(np.ascontiguousarray(raw)).to(gpu)
+    sd = None if sc is None else torch.from_numpy(np.ascontiguousarray(sc)).to(gpu)
+    y = torch.full((M, N), float("nan"), device=gpu)
+    args = (xd.data_ptr(), rd.data_ptr(), None if sd is None else sd.data_ptr(), y.data_ptr(), M, K, N)
+    if fmt in (MXFP8, MXFP4):
+        call("ccq_mx_linear_f32", *args, 0 if fmt == MXFP8 else 1, G or 32, float(s2), _dev.stream_ptr())
+    else:
+        call("ccq_fp8_linear_f32" if fmt == FP8_ROW else "ccq_int8_linear_f32", *args, _dev.stream_ptr())
+    return y.cpu().numpy()
+
+
+@pytest.mark.parametrize("fmt,G", FORMATS)
+@pytest.mark.parametrize("M,K,N", [(65, 256, 8300), (129, 512, 8200), (300, 768, 4100), (13, 320, 15130),
+                                   (70, 64, 3001), (200, 1088, 1030), (270, 832, 4099)])
+def test_tile_kernel_matches_oracle(gpu, fmt, G, M, K, N):
+    """The tiled kernel at each of its tile shapes (128 x 256, 128 x 128,
+    64 x 128), with part-filled rows and columns: in_features % 256 == 0 (two
+    activation parts, 1e-5 as above) and not (three parts, x exact: what is
+    left is float32 rounding of the sums, fewer than 32 of them in a row, at
+    2^-24 of a partial sum that stays within a few max|y| here)."""
+    rng = np.random.default_rng(7000 * fmt + 10 * G + M + K + N)
+    raw, sc, s2, w = _case(fmt, K, N, G, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    y = _apply(gpu, fmt, x, raw, sc, s2, N, G)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    tol = 1e-5 if K % 256 == 0 else 32 * 2.0 ** -24
+    assert np.all(np.isfinite(y))
+    assert np.max(np.abs(y - ref)) <= tol * np.max(np.abs(ref)), (fmt, G, M, K, N)
+
+
+def test_tile_kernel_non_finite_rows(gpu):
+    """Rows with Inf or NaN activations give what the float32 product gives
+    (three activation parts), and leave the other rows alone; a value above
+    the largest bf16 stays finite."""
+    rng = np.random.default_rng(3)
+    M, K, N = 70, 320, 3001
+    raw, sc, s2, w = _case(INT8_ROW, K, N, 0, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[3, 5], x[9, 7], x[11, 0] = np.inf, np.nan, np.float32(3.4e38)  # the last above the largest bf16
+    x[12, 1] = np.frombuffer(np.uint32(0x7F800001).tobytes(), np.float32)[0]  # NaN in its low bits only
+    y = _apply(gpu, INT8_ROW, x, raw, sc, s2, N, 0)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = x.astype(np.float64) @ oint8.dequant_row(raw.view(np.int8), sc).astype(np.float64).T
+    assert np.array_equal(np.isnan(y[[3, 9, 12]]), np.isnan(ref[[3, 9, 12]]))
+    assert np.array_equal(y[3][np.isinf(ref[3])], ref[3][np.isinf(ref[3])])
+    small = np.abs(ref[11]) < 1e38  # int8 products and the sum in float32 range before the row scale
+    assert np.isfinite(y[11][raw.view(np.int8)[:, 0] == 1]).all() and small.any()
+    rest = [i for i in range(M) if i not in (3, 9, 11, 12)]
+    assert np.max(np.abs(y[rest] - ref[rest])) <= 32 * 2.0 ** -24 * np.max(np.abs(ref[rest]))
