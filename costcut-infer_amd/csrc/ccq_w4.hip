@@ -1848,14 +1848,24 @@ size_t group_partials(int64_t M, int64_t K, int64_t N) {
 }
 }  // namespace
 
+namespace {
+// What every call with more than 64 rows of the grouped kernel's shapes brings:
+// row group sums, then the row ids of the 128-row tiles.
+size_t group_base_workspace(int64_t M, int64_t K) {
+  return align256((size_t)M * (size_t)(K / 128) * 4) + align256((size_t)cdiv(M, GG_BM) * GG_BM * 4);
+}
+}  // namespace
+
 extern "C" size_t ccq_w4_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size) {
   if (M <= 0 || K <= 0 || K % 128 || N <= 0 || !valid_group(group_size)) return 0;
-  if (w4_slab_takes(M, K, N, group_size)) return w4_slab_workspace(M, K, N);
-  if (!w4_grouped_takes(M, K, N, group_size)) return 0;
-  // row group sums, then the row ids of the 128-row tiles
-  // and the partial sums of a split K
-  return align256((size_t)M * (size_t)(K / 128) * 4) + align256((size_t)cdiv(M, GG_BM) * GG_BM * 4) +
-         group_partials(M, K, N);
+  // ... and the partial sums of a split K
+  const size_t base = w4_grouped_shape(M, K, N, group_size) ? group_base_workspace(M, K) : 0;
+  if (w4_grouped_takes(M, K, N, group_size)) return base + group_partials(M, K, N);
+  if (w4_slab_takes(M, K, N, group_size)) {
+    const size_t parts = w4_slab_workspace(M, K, N);
+    return parts > base ? parts : base;
+  }
+  return base;
 }
 
 extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, const uint32_t* sz, int scale_dtype,
@@ -1877,12 +1887,12 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
   CCQ_REQUIRE(x && w_tiled && sz && y, "ccq_w4_gemm: null pointer");
   CCQ_REQUIRE(aligned(x, 16) && aligned(w_tiled, 16) && aligned(sz, 16),
               "ccq_w4_gemm: x, w_tiled and sz must be 16-byte aligned");
+  const size_t base = w4_grouped_shape(M, K, N, group_size) ? group_base_workspace(M, K) : 0;
+  CCQ_REQUIRE(base == 0 || (workspace && workspace_bytes >= base && aligned(workspace, 256)),
+              "ccq_w4_gemm: workspace of %zu bytes (256-byte aligned) needed for M=%lld, %zu given",
+              ccq_w4_gemm_workspace_size(M, K, N, group_size), (long long)M, workspace_bytes);
   if (grouped) {
     // prefill-sized: 128-row tiles stream the weight once per tile
-    const size_t need = ccq_w4_gemm_workspace_size(M, K, N, group_size);
-    CCQ_REQUIRE(workspace && workspace_bytes >= need && aligned(workspace, 256),
-                "ccq_w4_gemm: workspace of %zu bytes (256-byte aligned) needed for M=%lld, %zu given", need,
-                (long long)M, workspace_bytes);
     CCQ_REQUIRE(M * K * 2 < (int64_t)1 << 32, "ccq_w4_gemm: activations of %lld x %lld exceed 4 GiB",
                 (long long)M, (long long)K);
     CCQ_REQUIRE(cdiv(M, GG_BM) * (N / 128) <= 0x7fffffff, "ccq_w4_gemm: M=%lld too large", (long long)M);
@@ -1911,9 +1921,9 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
     g.KT = (int)(K / 128);
     g.szw = (int)sz_words_per_column(K, group_size);
     g.nib_mask = 0x000F000Fu;
-    g.splits = group_splits(M, K, N);
+    g.splits = workspace_bytes >= base + group_partials(M, K, N) && aligned(y, 16) ? group_splits(M, K, N) : 1;
     if (g.splits > 1) {
-      g.y = (char*)rows + align256((size_t)tiles * GG_BM * 4);
+      g.y = (char*)workspace + base;
       g.y_dtype = CCQ_F32;
     }
     rc = launch_group_gemm<EPI_STORE>(g, x_dtype == CCQ_BF16, scale_dtype == CCQ_BF16, g.tiles, st);

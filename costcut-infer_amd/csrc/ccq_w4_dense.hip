@@ -406,8 +406,11 @@ size_t w4_slab_workspace(int64_t M, int64_t K, int64_t N) {
 
 int launch_w4_slab(const W4DenseP& d, void* workspace, size_t workspace_bytes, hipStream_t st) {
   SlabPlan pl = plan_slab(d.M, d.K, d.N);
-  // without the workspace one workgroup takes all of K
-  if (workspace == nullptr || workspace_bytes < w4_slab_workspace(d.M, d.K, d.N) || !aligned(workspace, 16)) pl.splits = 1;
+  // without the workspace (or with an output that takes no 16-byte stores) one
+  // workgroup takes all of K
+  if (workspace == nullptr || workspace_bytes < w4_slab_workspace(d.M, d.K, d.N) || !aligned(workspace, 16) ||
+      !aligned(d.y, 16))
+    pl.splits = 1;
   W4SlabP p = {};
   p.x = d.x;
   p.w = d.w;

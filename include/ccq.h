@@ -256,10 +256,11 @@ int64_t ccq_awq_sz_words(int64_t K, int64_t group_size);
 int ccq_awq_pack_sz(const int32_t* qzeros, const void* scales, int scale_dtype,
                     uint32_t* sz, int64_t K, int64_t N, int64_t group_size, void* stream);
 
-/* Workspace bytes ccq_w4_gemm needs for these sizes: 0 for the decode
- * kernels (M <= 64, or group_size != 128, or N % 128 != 0, or K < 256),
- * else the per-row group sums of x (M * K/128 floats) and the row ids of
- * the 128-row tiles, each 256-byte rounded. */
+/* Workspace bytes ccq_w4_gemm takes for these sizes: 0 up to 16 rows.  More
+ * than 64 rows of group 128, N % 128 == 0 and K >= 256 need at least the row
+ * group sums and row ids (a shorter workspace is an error); what is beyond
+ * those, and any workspace of other sizes, holds the partial sums of a split
+ * K, without which K is not split. */
 size_t ccq_w4_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size);
 
 /* y [M, N] = x [M, K] @ dequant(W) with fp32 accumulation.
@@ -267,11 +268,10 @@ size_t ccq_w4_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group
  * CCQ_F16 | CCQ_BF16; y_dtype CCQ_F16 | CCQ_BF16 | CCQ_F32.  w_tiled from
  * ccq_awq_repack, sz from ccq_awq_pack_sz.  group_size in {32, 64, 128}.
  * x, w_tiled and sz must be 16-byte aligned.  M <= 16 with group 128 and
- * K <= 4096: the persistent streaming kernel (weights read once); other
- * M <= 64: one workgroup per 16-row tile and column block (one weight pass
- * per 16 rows); no workspace for either.  Larger M with group 128,
- * N % 128 == 0 and K >= 256: the grouped MFMA kernel over 128-row tiles,
- * which needs ccq_w4_gemm_workspace_size bytes (256-byte aligned).
+ * K <= 4096: the persistent streaming kernel (weights read once).  Above:
+ * a 16-row kernel (one weight pass per 16 rows) while its workgroups fit the
+ * CUs, a 64-row kernel past that, and for the larger products of group 128,
+ * N % 128 == 0 and K >= 256 the grouped MFMA kernel over 128-row tiles.
  * Replaces WeightOnlyMethod.apply (quant/weight_only.py:37-54) for AWQ. */
 int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled,
                 const uint32_t* sz, int scale_dtype,
