@@ -22,7 +22,12 @@ def require_gpu() -> torch.device:
 
 
 def stream_ptr(device: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The hipStream_t of the device's current torch stream.  Callers hold a
+    tensor on the device, so torch is initialised; the raw query is 0.1 us,
+    ``torch.cuda.current_stream().cuda_stream`` 2.0-2.8 us of a decode call
+    that takes 5 us on the GPU."""
+    index = device.index if device is not None and device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def is_host(a) -> bool:
@@ -31,6 +36,9 @@ def is_host(a) -> bool:
 
 def to_device(a, dtype: torch.dtype | None = None) -> torch.Tensor:
     """numpy / bytes / torch -> contiguous tensor on the current GPU."""
+    if (isinstance(a, torch.Tensor) and a.is_cuda and (dtype is None or a.dtype == dtype) and a.is_contiguous()
+            and a.get_device() == torch.cuda.current_device()):
+        return a  # what the conversions below return for it, without their 1.9 us
     dev = require_gpu()
     if isinstance(a, (bytes, bytearray, memoryview)):
         a = np.frombuffer(a, dtype=np.uint8)

@@ -146,15 +146,16 @@ def gemm(x: torch.Tensor, w: AwqWeights, out_dtype: torch.dtype | None = None) -
     """``y = x @ dequant(W)`` with fp32 accumulation; x fp16/bf16 ``[M, K]``."""
     if x.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError(f"AWQ GEMM activations must be float16 or bfloat16, got {x.dtype}")
-    x2 = x.reshape(-1, x.shape[-1]).contiguous()
+    x2 = x if x.dim() == 2 and x.is_contiguous() else x.reshape(-1, x.shape[-1]).contiguous()
     M, K = x2.shape
     if K != w.K:
         raise ValueError(f"AWQ GEMM: x has {K} features, weight expects {w.K}")
     out_dtype = out_dtype or x.dtype
     y = torch.empty((M, w.N), dtype=out_dtype, device=x.device)
-    nbytes = lib().ccq_w4_gemm_workspace_size(M, K, w.N, w.group_size)
+    # up to 16 rows run in one launch without scratch memory
+    nbytes = lib().ccq_w4_gemm_workspace_size(M, K, w.N, w.group_size) if M > 16 else 0
     ws = _dev.workspace("w4_gemm", nbytes, x.device) if nbytes else None
     call("ccq_w4_gemm", x2.data_ptr(), _dev.DTYPE_CODE[x.dtype], w.w_tiled.data_ptr(), w.sz.data_ptr(),
          _scale_code(w.scale_dtype), y.data_ptr(), _dev.DTYPE_CODE[out_dtype], M, K, w.N, w.group_size,
          ws.data_ptr() if ws is not None else None, nbytes, _dev.stream_ptr(x.device))
-    return y.reshape(*x.shape[:-1], w.N)
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], w.N)
