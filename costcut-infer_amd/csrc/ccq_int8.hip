@@ -441,6 +441,104 @@ __global__ __launch_bounds__(256) void int8_gemm_big_kernel(const int8_t* __rest
     }
 }
 
+// Prefill GEMM for K % 128 == 0 (W8A8 M=1024 K=N=4096 49.4 -> 34.7 us, M=128
+// N=14336 47.7 -> 27.2, M=4096 380 -> 347 against the register-staged kernel
+// above, which stays for other K): 8 waves, 4 x 2 blocks of 32 RT x 64, so a tile
+// of 128 RT x 128.  K runs in 128-byte chunks through a ring of NS stages that
+// global_load_lds fills from HBM: two or three chunks are in flight during the
+// MFMAs, without registers or LDS stores of their own, and one barrier per
+// chunk publishes a stage and frees the one before.  LDS rows are 128 bytes,
+// 16-byte pieces XOR-swizzled by (row >> 1), so 16 rows of an operand read hit
+// 16 different bank groups.  Rows past M or N repeat the last one (not
+// stored).  Bound by the operand reads from LDS: 3 KiB per 2 MFMAs of a wave
+// at RT = 1, 4 KiB per 4 at RT = 2.
+template <int RT>
+__global__ __launch_bounds__(512, 2) void int8_gemm_ring_kernel(const int8_t* __restrict__ xq,
+                                                                const float* __restrict__ xs,
+                                                                const int8_t* __restrict__ w,
+                                                                const float* __restrict__ ws, float* __restrict__ y,
+                                                                int32_t* __restrict__ part, int M, int N, int K,
+                                                                int kper, int mtiles, int ntiles) {
+  constexpr int BM = 128 * RT, BN = 128, A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
+  constexpr int NS = RT == 1 ? 4 : 3;
+  constexpr int CA = BM / 64, CB = BN / 64, COPIES = CA + CB;  // copies (8 rows each) per wave and stage
+  __shared__ __align__(16) char smem[NS * STAGE];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1, r = lane & 31, h = lane >> 5;
+  // the row tiles of a column block are neighbours on one XCD
+  const int id = xcd_remap(blockIdx.x, gridDim.x), per = mtiles * ntiles, sp = id / per, q = id - sp * per;
+  const int m0 = (q % mtiles) * BM, n0 = (q / mtiles) * BN;
+  const int kb = sp * kper, S = (min(K, kb + kper) - kb) / 128;
+
+  uint32_t aoff[CA], boff[CB];
+  auto off = [&](int first, int c, int rows) {
+    const int row = 8 * c + (lane >> 3);
+    return (uint32_t)((int64_t)min(first + row, rows - 1) * K + (((lane & 7) ^ ((row >> 1) & 7)) * 16));
+  };
+#pragma unroll
+  for (int i = 0; i < CA; ++i) aoff[i] = off(m0, wave * CA + i, M);
+#pragma unroll
+  for (int i = 0; i < CB; ++i) boff[i] = off(n0, wave * CB + i, N);
+  const uint32_t lds0 = lds_addr(smem);
+  auto issue = [&](int i) {
+    const uint32_t st = lds0 + (i % NS) * STAGE;
+    const int k0 = kb + i * 128;
+#pragma unroll
+    for (int c = 0; c < CA; ++c) dma16(xq + k0, aoff[c], st + (wave * CA + c) * 1024);
+#pragma unroll
+    for (int c = 0; c < CB; ++c) dma16(w + k0, boff[c], st + A_BYTES + (wave * CB + c) * 1024);
+  };
+  i32x16 acc[RT][2];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = i32x16{};
+  auto frag = [&](const char* base, int row0, int s) {
+    return *reinterpret_cast<const i32x4v*>(base + (row0 + r) * 128 + (((2 * s + h) ^ ((r >> 1) & 7)) * 16));
+  };
+
+  for (int i = 0; i < NS - 1 && i < S; ++i) issue(i);
+  for (int i = 0; i < S; ++i) {
+    if (i + NS - 1 <= S)
+      wait_vmcnt<(NS - 2) * COPIES>();  // the NS - 2 chunks after i may stay in flight
+    else
+      wait_vmcnt<0>();
+    lds_barrier();
+    if (i + NS - 1 < S) issue(i + NS - 1);  // into the slot of chunk i - 1
+    const char* A = smem + (i % NS) * STAGE;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      i32x4v af[RT], bf[2];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) bf[c] = frag(A + A_BYTES, 64 * wn + 32 * c, s);
+#pragma unroll
+      for (int c = 0; c < RT; ++c) af[c] = frag(A, 32 * (wm * RT + c), s);
+#pragma unroll
+      for (int c = 0; c < RT; ++c)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[c][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[c], bf[j], acc[c][j], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int col = n0 + 64 * wn + 32 * j + r;
+    if (col >= N) continue;
+    const float wsc = ws[col];
+#pragma unroll
+    for (int c = 0; c < RT; ++c)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = m0 + 32 * (wm * RT + c) + 8 * (e >> 2) + 4 * h + (e & 3);
+        if (row >= M) continue;
+        if (part == nullptr)
+          y[(int64_t)row * N + col] = ((float)acc[c][j][e] * xs[row]) * wsc;
+        else
+          part[((int64_t)sp * M + row) * N + col] = acc[c][j][e];
+      }
+  }
+}
+
 __global__ void int8_splitk_epilogue_kernel(const int32_t* __restrict__ part, const float* __restrict__ xs,
                                             const float* __restrict__ ws, float* __restrict__ y, int M, int N,
                                             int splits) {
@@ -485,12 +583,24 @@ bool int8_big(int64_t M, int64_t K, int64_t N) {
   return M > I8_SKINNY_M && M * K < ((int64_t)1 << 31) && N * K < ((int64_t)1 << 31);
 }
 
+// the ring kernel (K % 128 == 0), and its tile height: 256 rows where those
+// tiles still cover the CUs
+bool int8_ring(int64_t M, int64_t K, int64_t N) { return int8_big(M, K, N) && K % 128 == 0; }
+int int8_ring_rt(int64_t M, int64_t N) { return cdiv(M, 256) * cdiv(N, 128) >= 256 ? 2 : 1; }
+
 int int8_splits(int64_t M, int64_t K, int64_t N) {
   if (K == 0 || K % 16 != 0) return 1;
   int64_t s = 1;
   if (int8_skinny(M, K, N)) {
     const int64_t waves = cdiv(N, 32) * 4;
     while (waves * s * 2 <= 2048 && K / (2 * s) >= 512 && s < 64) s *= 2;
+    return (int)s;
+  }
+  if (int8_ring(M, K, N)) {
+    // one workgroup per CU fills it: no more splits than give each CU one (M=1024
+    // K=N=4096 in two splits of 512 workgroups: 31 us and 13 more of partial sums)
+    const int64_t tiles = cdiv(M, 128 * int8_ring_rt(M, N)) * cdiv(N, 128);
+    while (tiles * s * 2 <= 256 && K / (2 * s) >= 512 && s < 64) s *= 2;
     return (int)s;
   }
   const int64_t bt = int8_big(M, K, N) ? BG_T : I8_BT;
@@ -564,6 +674,19 @@ extern "C" int ccq_int8_linear(const int8_t* xq, const float* x_scale, const int
     launch(int8_gemm_skinny_kernel<false>, dim3((unsigned)cdiv(N, 32), (unsigned)nsplit), dim3(256), 0,
                        st, xq, (const float*)nullptr, (float*)nullptr, x_scale, w, w_scale, y, (int32_t*)workspace,
                        (int)M, (int)N, K, kper);
+  } else if (int8_ring(M, K, N)) {
+    const int kper = (int)(cdiv(cdiv(K, s), 128) * 128), rt = int8_ring_rt(M, N);
+    nsplit = (int)cdiv(K, kper);
+    const int mt = (int)cdiv(M, 128 * rt), nt = (int)cdiv(N, 128);
+    CCQ_REQUIRE((int64_t)mt * nt * nsplit <= 0x7fffffff, "ccq_int8_linear: M=%lld too large", (long long)M);
+    const dim3 grid((unsigned)(mt * nt * nsplit));
+    int32_t* part = nsplit > 1 ? (int32_t*)workspace : nullptr;
+    if (rt == 2)
+      launch(int8_gemm_ring_kernel<2>, grid, dim3(512), 0, st, xq, x_scale, w, w_scale, y, part, (int)M, (int)N, (int)K,
+             kper, mt, nt);
+    else
+      launch(int8_gemm_ring_kernel<1>, grid, dim3(512), 0, st, xq, x_scale, w, w_scale, y, part, (int)M, (int)N, (int)K,
+             kper, mt, nt);
   } else if (int8_big(M, K, N)) {
     const int64_t kper = cdiv(cdiv(K, s), BG_KC) * BG_KC;
     const dim3 grid((unsigned)cdiv(N, BG_T), (unsigned)cdiv(M, BG_T), (unsigned)cdiv(K, kper));

@@ -143,3 +143,22 @@ def test_w8a8_fused_matches_two_kernels(gpu, M, K, N):
         y2 = int8_linear(xq2, xs2, w, s)
         assert np.array_equal(xs.cpu().numpy().view(np.uint32), xs2.cpu().numpy().view(np.uint32))
         assert _same(y.cpu().numpy(), y2.cpu().numpy())
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 128, 1), (129, 384, 257), (257, 4096, 33), (40, 1664, 130), (260, 256, 16500),
+                                   (128, 896, 512)])
+def test_int8_ring_kernel_exact(gpu, M, K, N):
+    """The prefill kernel of K % 128 == 0: one chunk, fewer chunks than its
+    ring, K split, part-filled rows and columns, and the 256-row tiles (260 x
+    16500).  Sums are whole numbers below 2^53, exact in float64, so y must be
+    bit-identical."""
+    from ccut.quant.int8 import int8_linear
+
+    rng = np.random.default_rng(M + K + N)
+    xq = rng.integers(-127, 128, (M, K)).astype(np.int8)
+    w = rng.integers(-127, 128, (N, K)).astype(np.int8)
+    xs = (rng.random(M) * 0.1 + 1e-3).astype(np.float32)
+    ws = (rng.random(N) * 0.02 + 1e-4).astype(np.float32)
+    y = int8_linear(*(torch.from_numpy(a).to(gpu) for a in (xq, xs, w, ws))).cpu().numpy()
+    acc = (xq.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32)
+    assert _same(y, acc * xs[:, None] * ws[None, :])
