@@ -249,7 +249,9 @@ int wq_mfma_linear(int fmt, const float* x, const uint8_t* w, const void* scale,
   const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
   const WqP p{x, w, scale, y, M, K, N, mx && scale ? group_size : 32, scale2};
   const bool g16 = mx && scale && group_size == 16;
-  const int rc = wq_tile_linear(fmt, p, g16, stream, name);
+  int rc = wq_tile_linear(fmt, p, g16, stream, name);
+  if (rc >= 0) return rc;
+  rc = wq_rows_linear(fmt, p, g16, stream, name);
   if (rc >= 0) return rc;
   if (K % WQ_KC != 0) return -1;
   switch (fmt) {

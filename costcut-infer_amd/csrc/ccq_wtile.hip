@@ -141,10 +141,12 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
     }
 #pragma unroll
     for (int j = 0; j < WPT / 8; ++j) {
-      float s = 1.f;
-      if constexpr (Tr::MX) s = e8m0_to_f32(sr[NSC == 2 ? j * 8 / G : 0] & 255u);
-      const bf16x8 b = FMT == WQ_MXFP4 ? wq_decode8<FMT>(wr[j], 0, s)
-                                       : wq_decode8<FMT>(wr[FMT == WQ_MXFP4 ? 0 : 2 * j], wr[FMT == WQ_MXFP4 ? 0 : 2 * j + 1], s);
+      bf16x8 b;
+      const uint32_t e = Tr::MX ? sr[NSC == 2 ? j * 8 / G : 0] & 255u : 0u;
+      if constexpr (FMT == WQ_MXFP4)
+        b = mx4_word_bf16(wr[j], mx4_lut(e));
+      else
+        b = wq_decode8<FMT>(wr[2 * j], wr[2 * j + 1], Tr::MX ? e8m0_to_f32(e) : 1.f);
       const int piece = wk / 8 + j;
       *reinterpret_cast<bf16x8*>(S + A_BYTES + wrow * 128 + ((piece ^ ((wrow >> 1) & 7)) * 16)) = b;
     }

@@ -87,6 +87,19 @@ def test_wq_matches_oracle(gpu, fmt, G, M, K, N):
 
 
 @pytest.mark.parametrize("fmt,G", FORMATS)
+@pytest.mark.parametrize("M,K,N", [(16, 768, 4101), (3, 2304, 8190), (13, 2304, 8300), (9, 4352, 8210)])
+def test_rows_kernel_wider_blocks(gpu, fmt, G, M, K, N):
+    """Up to 16 rows on 32- and 64-column workgroups: k-tile counts that leave
+    some of the 8 waves one more than others, part-filled last columns."""
+    rng = np.random.default_rng(300 * fmt + 10 * G + M + K + N)
+    raw, sc, s2, w = _case(fmt, K, N, G, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    y = _run(gpu, fmt, x, raw, sc, s2, N, G)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.max(np.abs(y - ref)) <= 1e-5 * np.max(np.abs(ref)), (fmt, G, M, K, N)
+
+
+@pytest.mark.parametrize("fmt,G", FORMATS)
 def test_wq_one_hot_is_exact(gpu, fmt, G):
     """x = identity: y[b, r] = W[r, b] bit for bit, so every code's decode
     and its scale (row or group) are checked through the MFMA path."""
