@@ -154,7 +154,8 @@ def gemm(x: torch.Tensor, w: AwqWeights, out_dtype: torch.dtype | None = None) -
     y = torch.empty((M, w.N), dtype=out_dtype, device=x.device)
     # up to 16 rows run in one launch without scratch memory
     nbytes = lib().ccq_w4_gemm_workspace_size(M, K, w.N, w.group_size) if M > 16 else 0
-    ws = _dev.workspace("w4_gemm", nbytes, x.device) if nbytes else None
+    # this call's own scratch, so that calls on several streams do not share it
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
     call("ccq_w4_gemm", x2.data_ptr(), _dev.DTYPE_CODE[x.dtype], w.w_tiled.data_ptr(), w.sz.data_ptr(),
          _scale_code(w.scale_dtype), y.data_ptr(), _dev.DTYPE_CODE[out_dtype], M, K, w.N, w.group_size,
          ws.data_ptr() if ws is not None else None, nbytes, _dev.stream_ptr(x.device))

@@ -138,6 +138,28 @@ def test_gemm_slab_kernel_row_blocks(gpu, M, K, N, G):
     assert _gemm_case(gpu, M, K, N, G, torch.bfloat16, torch.float32, seed=M) <= TIGHT
 
 
+def test_gemm_split_k_on_two_streams(gpu):
+    """Calls whose K is split keep their partial sums apart: two streams
+    without an order between them give what one stream gives."""
+    from ccut.quant import awq
+
+    M, K, N, G = 33, 4480, 6160, 128
+    qw, qz, s = _make(K, N, G, 9)
+    w = awq.prepare(torch.from_numpy(qw).to(gpu), torch.from_numpy(qz).to(gpu), torch.from_numpy(s).to(gpu), G)
+    g = torch.Generator().manual_seed(9)
+    xs = [torch.randn((M, K), generator=g).to(torch.float16).to(gpu) for _ in range(2)]
+    ref = [awq.gemm(x, w) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    out = [[], []]
+    for _ in range(8):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                out[i].append(awq.gemm(xs[i], w))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, ref[i]) for i in range(2) for y in out[i])
+
+
 def test_gemm_slab_kernel_without_workspace(gpu):
     """A caller that passes no workspace gets the unsplit kernel, equal up to
     the order of the float32 sums."""
