@@ -144,9 +144,13 @@ __global__ __launch_bounds__(512, 2) void wq_rows_kernel(const WqP p) {
 template <int FMT, bool G16>
 void launch_rows(const WqP& p, int nb, hipStream_t st) {
   const dim3 grid((unsigned)cdiv(p.N, 16 * nb)), block(512);
-  if (nb == 4)
-    launch((wq_rows_kernel<FMT, G16, 4>), grid, block, 0, st, p);
-  else if (nb == 2)
+  if constexpr (FMT == WQ_MXFP4) {
+    if (nb == 4) {
+      launch((wq_rows_kernel<FMT, G16, 4>), grid, block, 0, st, p);
+      return;
+    }
+  }
+  if (nb == 2)
     launch((wq_rows_kernel<FMT, G16, 2>), grid, block, 0, st, p);
   else
     launch((wq_rows_kernel<FMT, G16, 1>), grid, block, 0, st, p);
@@ -158,15 +162,14 @@ int wq_rows_linear(int fmt, const WqP& p, bool g16, hipStream_t st, const char* 
   if (p.M > 16 || p.K % 256 != 0 || cdiv(p.N, 64) > 256) return -1;
   // the fewest columns per workgroup whose workgroups are one round of the CUs
   const int nb = cdiv(p.N, 16) <= 256 ? 1 : (cdiv(p.N, 32) <= 256 ? 2 : 4);
-  // With 64 columns the 64-row kernel keeps the few-row batches of the one-byte
-  // formats (K=4096 N=14336: int8 M=8 16.9 us against 17.9, M=16 18.7 against
-  // 18.3; fp8 M=4 17.1 against 17.4, M=16 20.0 against 18.0; MXFP8 M=4 21.5
-  // against 22.1, M=16 26.1 against 23.8; MXFP4 M=1 19.4 -> 16.5, M=16 21.6 ->
-  // 17.5; 32 columns, K=6144 N=8192 M=16: fp8 27.4 -> 14.9, MXFP4 29.8 -> 14.5)
-  // and short K, where a wave has no third k-tile to load ahead (K=2048 N=9000
-  // M=16: fp8 11.8 us against 12.7, MXFP8 14.2 against 15.6; MXFP4 13.0 -> 11.5,
-  // but K=1024 N=12000 9.9 against 10.8).
-  if (nb == 4 && (fmt == WQ_MXFP4 ? p.K < 2048 : p.M <= 8 || p.K <= 2048)) return -1;
+  // With 64 columns the 64-row kernel keeps the one-byte formats: K=4096 N=14336
+  // M=16, weights from HBM (12 sets in turn), fp8 20.7 us against 22.9 and MXFP8
+  // 27.0 against 28.2 (from the Infinity Cache 20.0 against 18.0 and 26.1
+  // against 23.8); MXFP4 20.7 -> 17.4 at M=1 and 23.5 -> 18.8 at M=16.  And short
+  // K, where a wave has no third k-tile to load ahead (MXFP4 K=1024 N=12000 9.9
+  // against 10.8, K=2048 N=9000 13.0 -> 11.5).  32 columns: K=6144 N=8192 M=16
+  // fp8 27.4 -> 14.9, MXFP4 29.8 -> 14.5.
+  if (nb == 4 && (fmt != WQ_MXFP4 || p.K < 2048)) return -1;
   switch (fmt) {
     case WQ_FP8_ROW: launch_rows<WQ_FP8_ROW, false>(p, nb, st); break;
     case WQ_INT8_ROW: launch_rows<WQ_INT8_ROW, false>(p, nb, st); break;
