@@ -25,7 +25,11 @@ def stream_ptr(device: torch.device | None = None) -> int:
     """The hipStream_t of the device's current torch stream.  Callers hold a
     tensor on the device, so torch is initialised; the raw query is 0.1 us,
     ``torch.cuda.current_stream().cuda_stream`` 2.0-2.8 us of a decode call
-    that takes 5 us on the GPU."""
+    that takes 5 us on the GPU.  A device that is no GPU is refused, as
+    ``current_stream`` does: for the calls that take ``x`` as it comes this is
+    what keeps a host pointer from a kernel."""
+    if device is not None and device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index if device is not None and device.index is not None else torch.cuda.current_device()
     return torch._C._cuda_getCurrentRawStream(index)
 
