@@ -19,12 +19,21 @@
 // Activation parts: two (x = hi + lo, |x - hi - lo| <= 2^-17 |x|, as the
 // 64-row kernel) where in_features % 256 == 0; three otherwise, since those
 // shapes otherwise run on the float32 streaming kernels: truncations to 8 bits
-// each, so that x = hi + mid + lo exactly.
+// each, so that x = hi + mid + lo exactly down to |x| = 2^-110 (below, what is
+// under bf16's smallest step 2^-133 is lost).
+//
+// Weights are exact in bf16 except MXFP8 codes under the E8M0 bytes 1 and 2
+// (scales 2^-126 and 2^-125), which reach below bf16's smallest step 2^-133.
+// With three parts (the float32 kernels took those shapes) a workgroup that
+// meets such a byte runs its chunks again with what the rounding left over,
+// times 2^64 (wq_tiny8); others pay an OR per scale byte.
 //
 // Sums: the MFMAs add up 128 k, and these spans are added on the VALU: K / 16
 // dependent roundings in one chain would cost more than the parts do (K=2176:
 // 4.3e-7 relative against 64 bits in one chain, the streaming kernels 1.3e-7).
 #include "ccq_wq.h"
+
+#include <type_traits>
 
 namespace ccq {
 
@@ -32,8 +41,8 @@ namespace {
 
 constexpr int WT_KC = 64;
 
-// 8 floats -> NSP bf16 pieces of 16 bytes
-template <int NSP>
+// 8 floats -> NSP bf16 pieces of 16 bytes (FIN, three parts: Inf and NaN -> 0)
+template <int NSP, bool FIN = false>
 __device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[NSP]) {
   if constexpr (NSP == 2) {
 #pragma unroll
@@ -51,7 +60,7 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[NSP]) {
       const float r = fin ? v[e] - __uint_as_float(u & 0xffff0000u) : 0.f;
       const uint32_t ur = __float_as_uint(r);
       // a NaN stays one when its low bits go
-      p[0][e] = !fin && (u & 0x007fffffu) ? u | 0x00400000u : u;
+      p[0][e] = FIN && !fin ? 0u : (!fin && (u & 0x007fffffu) ? u | 0x00400000u : u);
       p[1][e] = ur;
       p[2][e] = __float_as_uint(r - __uint_as_float(ur & 0xffff0000u));
     }
@@ -60,6 +69,23 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[NSP]) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[q][j] = __builtin_amdgcn_perm(p[q][2 * j + 1], p[q][2 * j], 0x07060302u);
   }
+}
+
+// Eight MXFP8 weights under the scale byte 1 or 2: rounded to bf16, but never to
+// zero (Inf times a weight that is not zero is no NaN), or (LEFT) 2^64 times
+// what that leaves, at most three steps of 2^-135: exact.
+template <bool LEFT>
+__device__ __forceinline__ bf16x8 wq_tiny8(uint32_t w0, uint32_t w1, uint32_t e) {
+  const float s = e8m0_to_f32(e);
+  float o[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float v = fp8_e4m3_to_f32(((j < 4 ? w0 : w1) >> (8 * (j & 3))) & 0xFFu) * s;
+    uint32_t h = f32_to_bf16_bits(v);
+    if (!(h & 0x7FFFu) && v != 0.f) h |= 1u;
+    o[j] = LEFT ? (v - bf16_bits_to_f32(h)) * 0x1p64f : bf16_bits_to_f32(h);
+  }
+  return pack_bf16x8(o);
 }
 
 // WM x WN waves, each RT x CT tiles of 32 x 32; NSP activation parts.
@@ -73,6 +99,7 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
   constexpr int WW = WPT / Tr::KDIV / 4;       // ... in 32-bit words
   constexpr int TPR = WT_KC / WPT;             // threads per weight row
   constexpr int NSC = Tr::MX ? (WPT > (G16 ? 16 : 32) ? 2 : 1) : 0;
+  constexpr bool TINY = FMT == WQ_MXFP8 && NSP == 3;
   static_assert(WM * WN == 8 && XP >= 1 && (WPT == 16 || WPT == 32) && 2 * BUF <= 160 * 1024, "tile shape");
   __shared__ __align__(16) char smem[2 * BUF];
 
@@ -129,13 +156,15 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
       for (int j = 0; j < NSC; ++j) sr[j] = has_sc ? sp[(int64_t)c * (WT_KC / G) + j] : 127u;
     }
   };
-  auto store = [&](int buf) {
+  bool tiny = false;  // a scale byte 1 or 2 in this thread's weights
+  auto store = [&](int buf, auto left_c) {
+    constexpr bool LEFT = decltype(left_c)::value;
     char* S = smem + buf * BUF;
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
       const float v[8] = {xr[i][0].x, xr[i][0].y, xr[i][0].z, xr[i][0].w, xr[i][1].x, xr[i][1].y, xr[i][1].z, xr[i][1].w};
       u32x4 o[NSP];
-      split8<NSP>(v, o);
+      split8<NSP, LEFT>(v, o);
 #pragma unroll
       for (int q = 0; q < NSP; ++q) *reinterpret_cast<u32x4*>(S + q * A_PART + xd[i]) = o[q];
     }
@@ -145,8 +174,13 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
       const uint32_t e = Tr::MX ? sr[NSC == 2 ? j * 8 / G : 0] & 255u : 0u;
       if constexpr (FMT == WQ_MXFP4)
         b = mx4_word_bf16(wr[j], mx4_lut(e));
+      else if (TINY && e - 1u < 2u)
+        b = wq_tiny8<LEFT>(wr[2 * j], wr[2 * j + 1], e);
+      else if constexpr (LEFT)
+        b = bf16x8{};
       else
         b = wq_decode8<FMT>(wr[2 * j], wr[2 * j + 1], Tr::MX ? e8m0_to_f32(e) : 1.f);
+      if constexpr (TINY) tiny |= e - 1u < 2u;
       const int piece = wk / 8 + j;
       *reinterpret_cast<bf16x8*>(S + A_BYTES + wrow * 128 + ((piece ^ ((wrow >> 1) & 7)) * 16)) = b;
     }
@@ -163,13 +197,13 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
       t[r][c] = f32x16{};
       if constexpr (NSP == 3) small[r][c] = f32x16{};
     }
-  auto fold = [&](f32x16 (&v)[RT][CT]) {
+  auto fold = [&](f32x16 (&a)[RT][CT], f32x16 (&v)[RT][CT], float f) {
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int c = 0; c < CT; ++c) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[r][c][i] += v[r][c][i];
+        for (int i = 0; i < 16; ++i) a[r][c][i] += v[r][c][i] * f;
         v[r][c] = f32x16{};
       }
   };
@@ -204,18 +238,27 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
     }
   };
 
-  load(0);
-  store(0);
-  lds_barrier();
-  for (int c = 0; c < nch; ++c) {
-    if (c + 1 < nch) load(c + 1);
-    multiply(c & 1);
-    if ((c & 1) || c + 1 == nch) fold(t);
-    if (c + 1 < nch) store((c + 1) & 1);  // last read in chunk c - 1, before the last barrier
+  auto chunks = [&](auto left_c, auto&& span_done) {
+    load(0);
+    store(0, left_c);
     lds_barrier();
-  }
+    for (int c = 0; c < nch; ++c) {
+      if (c + 1 < nch) load(c + 1);
+      multiply(c & 1);
+      if ((c & 1) || c + 1 == nch) span_done();
+      if (c + 1 < nch) store((c + 1) & 1, left_c);  // last read in chunk c - 1, before the last barrier
+      lds_barrier();
+    }
+  };
+  chunks(std::false_type{}, [&] { fold(acc, t, 1.f); });
 
-  if constexpr (NSP == 3) fold(small);
+  if constexpr (NSP == 3) fold(acc, small, 1.f);
+  if constexpr (TINY) {
+    if (__syncthreads_or(tiny)) {
+      chunks(std::true_type{}, [&] { fold(small, t, 1.f); });
+      fold(acc, small, 0x1p-64f);
+    }
+  }
 
   // register i of a tile: row 8 (i / 4) + 4 h + i % 4, column c32
 #pragma unroll

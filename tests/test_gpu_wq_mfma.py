@@ -217,3 +217,33 @@ def test_tile_kernel_non_finite_rows(gpu):
     assert np.isfinite(y[11][raw.view(np.int8)[:, 0] == 1]).all() and small.any()
     rest = [i for i in range(M) if i not in (3, 9, 11, 12)]
     assert np.max(np.abs(y[rest] - ref[rest])) <= 32 * 2.0 ** -24 * np.max(np.abs(ref[rest]))
+
+
+@pytest.mark.parametrize("G", [16, 32])
+@pytest.mark.parametrize("M,K,N", [(70, 320, 3001), (260, 320, 7000)])
+def test_tile_kernel_smallest_mx_scales(gpu, G, M, K, N):
+    """E8M0 bytes 1 and 2: products with e4m3 codes reach 2^-135, below bf16's
+    smallest step 2^-133, so the tiled kernel adds what its bf16 weights leave
+    out (three-part activations, K % 256 != 0; both tile sizes).  Columns of
+    only such groups, of only larger scales, and mixed, each within 32
+    roundings (as above) of its own largest value; Inf times a tiny weight
+    keeps its sign."""
+    rng = np.random.default_rng(G + M)
+    codes = rng.integers(0, 256, (N, K)).astype(np.uint8)
+    codes[(codes & 0x7F) == 0x7F] = 0x38
+    codes[codes & 0x78 == 0] |= 1  # subnormal codes, none zero (0 * Inf)
+    codes[:, : K // 2] &= 0x8F  # half of all columns: subnormal and smallest normal codes
+    codes[codes & 0x7F == 0] = 0x01
+    sc = np.where(rng.random((N, K // G)) < 0.5, 1, 2).astype(np.uint8)
+    sc[N // 3: 2 * N // 3] = 120
+    sc[2 * N // 3:, ::2] = 5
+    x = np.ldexp(rng.standard_normal((M, K)), 40).astype(np.float32)
+    w = omx.dequant_mxfp8(codes, sc.reshape(-1), G)
+    y = _apply(gpu, MXFP8, x, codes, sc, 1.0, N, G)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    err = np.max(np.abs(y - ref), axis=0) / np.max(np.abs(ref), axis=0)
+    assert np.max(err) <= 32 * 2.0 ** -24
+    x[3, 5], x[4, K // 2] = np.inf, -np.inf
+    y = _apply(gpu, MXFP8, x, codes, sc, 1.0, N, G)
+    assert np.array_equal(y[3], np.where(w[:, 5] > 0, np.inf, -np.inf))
+    assert np.array_equal(y[4], np.where(w[:, K // 2] > 0, -np.inf, np.inf))
