@@ -17,6 +17,16 @@ namespace {
 
 constexpr int WS_LD = 128 + 8;  // LDS row stride in bf16: rows 4 banks apart
 
+// Lanes of one wave hand each other values through LDS: the hardware keeps a
+// wave's LDS accesses in order, and the fences keep the compiler from moving
+// them across (to a lane the other lanes' addresses are unrelated ones; the
+// wave barrier alone only bounds the scheduling).  They emit no instruction.
+__device__ __forceinline__ void lane_exchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int FMT, bool G16, int NB>
 __global__ __launch_bounds__(512, 2) void wq_rows_kernel(const WqP p) {
   using Tr = WqTraits<FMT>;
@@ -81,15 +91,14 @@ __global__ __launch_bounds__(512, 2) void wq_rows_kernel(const WqP p) {
       *reinterpret_cast<u32x2*>(&xs[wave][0][row][k]) = u32x2{h01, h23};
       *reinterpret_cast<u32x2*>(&xs[wave][1][row][k]) = u32x2{l01, l23};
     }
-    // the wave's own LDS accesses are in order; only the compiler has to keep them
-    __builtin_amdgcn_wave_barrier();
+    lane_exchange();
     bf16x8 ah[4], al[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       ah[i] = *reinterpret_cast<const bf16x8*>(&xs[wave][0][c16][32 * q + 8 * i]);
       al[i] = *reinterpret_cast<const bf16x8*>(&xs[wave][1][c16][32 * q + 8 * i]);
     }
-    __builtin_amdgcn_wave_barrier();
+    lane_exchange();
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
