@@ -80,6 +80,8 @@ SIGNATURES: dict[str, tuple] = {
     "ccq_int8_linear_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     "ccq_int8_dequant": (_int, [_vp, _vp, _vp, _i64, _i64, _vp]),
     "ccq_int8_act_quant": (_int, [_vp, _vp, _vp, _i64, _i64, _vp]),
+    "ccq_wq_linear_kernel": (_int, [_int, _i64, _i64, _i64, _int, ctypes.POINTER(_int), ctypes.POINTER(_int)]),
+    "ccq_int8_linear_kernel": (_int, [_i64, _i64, _i64]),
     "ccq_int8_linear_workspace_size": (_sz, [_i64, _i64, _i64]),
     "ccq_int8_linear": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp]),
     "ccq_int8_w8a8_workspace_size": (_sz, [_i64, _i64, _i64]),
@@ -102,6 +104,7 @@ SIGNATURES: dict[str, tuple] = {
     "ccq_awq_unpack_tiled": (_int, [_vp, _vp, _i64, _i64, _vp]),
     "ccq_awq_sz_words": (_i64, [_i64, _i64]),
     "ccq_awq_pack_sz": (_int, [_vp, _vp, _int, _vp, _i64, _i64, _i64, _vp]),
+    "ccq_w4_gemm_kernel": (_int, [_i64, _i64, _i64, _i64]),
     "ccq_w4_gemm_workspace_size": (_sz, [_i64, _i64, _i64, _i64]),
     "ccq_w4_gemm": (_int, [_vp, _int, _vp, _vp, _int, _vp, _int, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
     "ccq_topk_softmax": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),

@@ -640,6 +640,13 @@ extern "C" int ccq_int8_act_quant(const float* x, int8_t* xq, float* x_scale, in
   return launch_status("ccq_int8_act_quant");
 }
 
+extern "C" int ccq_int8_linear_kernel(int64_t M, int64_t K, int64_t N) {
+  if (M <= 0 || K <= 0 || N <= 0 || K % 16 != 0) return 0;
+  if (int8_skinny(M, K, N)) return 1;
+  if (int8_ring(M, K, N)) return 1 + int8_ring_rt(M, N);
+  return int8_big(M, K, N) ? 4 : 5;
+}
+
 extern "C" size_t ccq_int8_linear_workspace_size(int64_t M, int64_t K, int64_t N) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
   const int s = int8_splits(M, K, N);

@@ -1856,6 +1856,26 @@ size_t group_base_workspace(int64_t M, int64_t K) {
 }
 }  // namespace
 
+namespace {
+// The kernel of a dense call; nq: quads per job of the streaming kernel.
+enum W4Route { W4_STREAM = 0, W4_SKINNY = 1, W4_SLAB = 2, W4_GROUPED = 3 };
+W4Route w4_gemm_route(int64_t M, int64_t K, int64_t N, int64_t G, int& nq) {
+  if (w4_grouped_takes(M, K, N, G)) return W4_GROUPED;
+  // 16-column jobs (one quad) when 32-column jobs would leave CUs idle
+  // (K=2048 N=5632: 176 jobs of 32 columns, 352 of 16)
+  nq = stream_nq(EPI_STORE, N, K, G);
+  if (nq == 2 && N / 32 < device_cus() && K <= 4096) nq = 1;
+  if (M <= 16 && nq > 0) return W4_STREAM;  // decode: one 16-row tile, weights streamed once
+  return w4_slab_takes(M, K, N, G) ? W4_SLAB : W4_SKINNY;
+}
+}  // namespace
+
+extern "C" int ccq_w4_gemm_kernel(int64_t M, int64_t K, int64_t N, int64_t group_size) {
+  int nq;
+  if (M <= 0 || K <= 0 || K % 128 || N <= 0 || N % 16 || !valid_group(group_size)) return -1;
+  return w4_gemm_route(M, K, N, group_size, nq);
+}
+
 extern "C" size_t ccq_w4_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size) {
   if (M <= 0 || K <= 0 || K % 128 || N <= 0 || !valid_group(group_size)) return 0;
   // ... and the partial sums of a split K
@@ -1880,8 +1900,9 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
   CCQ_REQUIRE(y_dtype == CCQ_F16 || y_dtype == CCQ_BF16 || y_dtype == CCQ_F32, "ccq_w4_gemm: bad y_dtype");
   CCQ_REQUIRE(K <= (1 << 20) && N / 16 <= 0x7fffffff, "ccq_w4_gemm: K=%lld or N=%lld too large", (long long)K,
               (long long)N);
-  const bool grouped = w4_grouped_takes(M, K, N, group_size);
-  CCQ_REQUIRE(grouped || cdiv(M, 16) <= 65535, "ccq_w4_gemm: M=%lld too large", (long long)M);
+  int nq = 0;
+  const W4Route route = K > 0 && N > 0 ? w4_gemm_route(M, K, N, group_size, nq) : W4_SKINNY;
+  CCQ_REQUIRE(route == W4_GROUPED || cdiv(M, 16) <= 65535, "ccq_w4_gemm: M=%lld too large", (long long)M);
   if (M == 0 || N == 0) return 0;
   CCQ_REQUIRE(K > 0, "ccq_w4_gemm: K == 0");
   CCQ_REQUIRE(x && w_tiled && sz && y, "ccq_w4_gemm: null pointer");
@@ -1891,7 +1912,7 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
   CCQ_REQUIRE(base == 0 || (workspace && workspace_bytes >= base && aligned(workspace, 256)),
               "ccq_w4_gemm: workspace of %zu bytes (256-byte aligned) needed for M=%lld, %zu given",
               ccq_w4_gemm_workspace_size(M, K, N, group_size), (long long)M, workspace_bytes);
-  if (grouped) {
+  if (route == W4_GROUPED) {
     // prefill-sized: 128-row tiles stream the weight once per tile
     CCQ_REQUIRE(M * K * 2 < (int64_t)1 << 32, "ccq_w4_gemm: activations of %lld x %lld exceed 4 GiB",
                 (long long)M, (long long)K);
@@ -1931,12 +1952,7 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
     return launch_w4_split_sum((const float*)g.y, y, y_dtype, g.splits, M * N, st);
   }
   const int64_t szw_d = sz_words_per_column(K, group_size);
-  // 16-column jobs (one quad) when 32-column jobs would leave CUs idle
-  // (K=2048 N=5632: 176 jobs of 32 columns, 352 of 16)
-  int nq = stream_nq(EPI_STORE, N, K, group_size);
-  if (nq == 2 && N / 32 < device_cus() && K <= 4096) nq = 1;
-  if (M <= 16 && nq > 0) {
-    // decode: one 16-row tile, weights streamed once
+  if (route == W4_STREAM) {
     W4SP w = {};
     w.x = x;
     w.ldx = K;
@@ -1955,7 +1971,7 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
     w.nib_mask = 0x000F000Fu;
     return launch_stream<EPI_STORE>(w, nq, x_dtype == CCQ_BF16, scale_dtype == CCQ_BF16, 1, as_stream(stream));
   }
-  if (w4_slab_takes(M, K, N, group_size)) {
+  if (route == W4_SLAB) {
     const W4DenseP d = {x, (const uint32_t*)w_tiled, sz, y, x_dtype == CCQ_BF16, scale_dtype == CCQ_BF16, y_dtype,
                         M, K, N, group_size};
     return launch_w4_slab(d, workspace, workspace_bytes, as_stream(stream));

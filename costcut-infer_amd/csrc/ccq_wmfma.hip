@@ -669,6 +669,24 @@ int moe_fp8row_ffn(const float* x, const int64_t* ids, const float* weights, voi
 
 using namespace ccq;
 
+extern "C" int ccq_wq_linear_kernel(int fmt, int64_t batch, int64_t in_features, int64_t out_features, int group_size,
+                                    int* tile_rows, int* tile_cols) {
+  int bm = 0, bn = 0, kernel = 0;
+  if (fmt >= WQ_FP8_ROW && fmt <= WQ_MXFP4 && batch > 0 && in_features > 0 && out_features > 0) {
+    const bool g16 = fmt >= WQ_MXFP8 && group_size == 16;
+    if (wq_tile_route(fmt, batch, in_features, out_features, bm, bn)) {
+      kernel = 3;
+    } else if (const int nb = wq_rows_route(fmt, g16, batch, in_features, out_features)) {
+      kernel = 2, bm = 16, bn = 16 * nb;
+    } else if (in_features % WQ_KC == 0) {
+      kernel = 1, bm = batch <= 16 ? 16 : (batch <= 32 ? 32 : 64), bn = WQ_COLS;
+    }
+  }
+  if (tile_rows) *tile_rows = kernel ? bm : 0;
+  if (tile_cols) *tile_cols = kernel ? bn : 0;
+  return kernel;
+}
+
 extern "C" int ccq_wq_mfma_linear_f32(const float* x, const uint8_t* w, const void* scale, float* y, int64_t batch,
                                       int64_t in_features, int64_t out_features, int fmt, int group_size,
                                       float scale2, void* stream) {

@@ -106,9 +106,13 @@ __device__ __forceinline__ bf16x8 wq_decode(const u32x4 (&wr)[WqTraits<FMT>::WB]
     return wq_decode8<FMT>(wr[i >> 1][(i & 1) * 2], wr[i >> 1][(i & 1) * 2 + 1], s);
 }
 
-// The form for up to 16 rows; -1 when it does not take the shape.
+// The form for up to 16 rows: its 16-column tiles per workgroup, 0 for shapes it
+// does not take (the launch: -1).
+int wq_rows_route(int fmt, bool g16, int64_t M, int64_t K, int64_t N);
 int wq_rows_linear(int fmt, const WqP& p, bool g16, hipStream_t st, const char* name);
-// The tiled form for many rows; -1 when it does not take the shape.
+// The tiled form for many rows: its tile, false for shapes it does not take
+// (the launch: -1).
+bool wq_tile_route(int fmt, int64_t M, int64_t K, int64_t N, int& bm, int& bn);
 int wq_tile_linear(int fmt, const WqP& p, bool g16, hipStream_t st, const char* name);
 
 }  // namespace ccq

@@ -167,10 +167,10 @@ void launch_rows(const WqP& p, int nb, hipStream_t st) {
 
 }  // namespace
 
-int wq_rows_linear(int fmt, const WqP& p, bool g16, hipStream_t st, const char* name) {
-  if (p.M > 16 || p.K % 256 != 0 || cdiv(p.N, 64) > 256) return -1;
+int wq_rows_route(int fmt, bool g16, int64_t M, int64_t K, int64_t N) {
+  if (M > 16 || K % 256 != 0 || cdiv(N, 64) > 256) return 0;
   // the fewest columns per workgroup whose workgroups are one round of the CUs
-  const int nb = cdiv(p.N, 16) <= 256 ? 1 : (cdiv(p.N, 32) <= 256 ? 2 : 4);
+  const int nb = cdiv(N, 16) <= 256 ? 1 : (cdiv(N, 32) <= 256 ? 2 : 4);
   // With 64 columns the 64-row kernel keeps the one-byte formats: K=4096 N=14336
   // M=16, weights from HBM (12 sets in turn), fp8 20.7 us against 22.9 and MXFP8
   // 27.0 against 28.2 (from the Infinity Cache 20.0 against 18.0 and 26.1
@@ -178,7 +178,13 @@ int wq_rows_linear(int fmt, const WqP& p, bool g16, hipStream_t st, const char* 
   // K, where a wave has no third k-tile to load ahead (MXFP4 K=1024 N=12000 9.9
   // against 10.8, K=2048 N=9000 13.0 -> 11.5).  32 columns: K=6144 N=8192 M=16
   // fp8 27.4 -> 14.9, MXFP4 29.8 -> 14.5.
-  if (nb == 4 && (fmt != WQ_MXFP4 || p.K < 2048)) return -1;
+  if (nb == 4 && (fmt != WQ_MXFP4 || K < 2048)) return 0;
+  return nb;
+}
+
+int wq_rows_linear(int fmt, const WqP& p, bool g16, hipStream_t st, const char* name) {
+  const int nb = wq_rows_route(fmt, g16, p.M, p.K, p.N);
+  if (nb == 0) return -1;
   switch (fmt) {
     case WQ_FP8_ROW: launch_rows<WQ_FP8_ROW, false>(p, nb, st); break;
     case WQ_INT8_ROW: launch_rows<WQ_INT8_ROW, false>(p, nb, st); break;

@@ -298,25 +298,31 @@ void launch_tile(const WqP& p, int bm, int bn, hipStream_t st) {
 
 }  // namespace
 
-int wq_tile_linear(int fmt, const WqP& p, bool g16, hipStream_t st, const char* name) {
-  if (p.K % WT_KC != 0) return -1;
-  if (p.K % 256 == 0) {
+bool wq_tile_route(int fmt, int64_t M, int64_t K, int64_t N, int& bm, int& bn) {
+  if (K % WT_KC != 0) return false;
+  if (K % 256 == 0) {
     // the 64-row kernel is as fast while its 64 x 64 blocks are one round of
     // the CUs (fp8 M=512 K=N=2048 26 us against 28; MXFP4 25 against 33); past
     // that fp8 K=4096 N=14336 M=65 79 -> 47 us, M=128 97 -> 49, M=512 332 -> 129
-    if (p.M <= 64 || cdiv(p.M, 64) * cdiv(p.N, 64) <= 256) return -1;
-  } else if (p.M <= 12 || p.M * p.N < (fmt >= WQ_MXFP8 ? 1 << 17 : 3 << 16)) {
+    if (M <= 64 || cdiv(M, 64) * cdiv(N, 64) <= 256) return false;
+  } else if (M <= 12 || M * N < (fmt >= WQ_MXFP8 ? 1 << 17 : 3 << 16)) {
     // a workgroup takes about 1 us per chunk however few there are, the
     // streaming kernels a time in proportion to M N (K=2176 N=4001 M=33: int8
     // 36.6 us against 37.6, MXFP4 62 against 44; K=4224 N=14336: int8 M=10 52
     // against 68, M=16 79 against 68, M=64 310 -> 70, M=512 2506 -> 241)
-    return -1;
+    return false;
   }
   // the largest tile that still gives most CUs one
-  int bm = 128, bn = p.K % 256 == 0 ? 256 : 128;
-  if (cdiv(p.M, bm) * cdiv(p.N, bn) < 160) bn = 128;
-  if (cdiv(p.M, bm) * cdiv(p.N, bn) < 160) bm = 64;
-  if (cdiv(p.M, bm) * cdiv(p.N, bn) > 0x7fffffff) return -1;
+  bm = 128;
+  bn = K % 256 == 0 ? 256 : 128;
+  if (cdiv(M, bm) * cdiv(N, bn) < 160) bn = 128;
+  if (cdiv(M, bm) * cdiv(N, bn) < 160) bm = 64;
+  return cdiv(M, bm) * cdiv(N, bn) <= 0x7fffffff;
+}
+
+int wq_tile_linear(int fmt, const WqP& p, bool g16, hipStream_t st, const char* name) {
+  int bm, bn;
+  if (!wq_tile_route(fmt, p.M, p.K, p.N, bm, bn)) return -1;
   switch (fmt) {
     case WQ_FP8_ROW: launch_tile<WQ_FP8_ROW, false>(p, bm, bn, st); break;
     case WQ_INT8_ROW: launch_tile<WQ_INT8_ROW, false>(p, bm, bn, st); break;

@@ -210,6 +210,20 @@ int ccq_wq_mfma_linear_f32(const float* x, const uint8_t* w, const void* scale,
                            int64_t out_features, int fmt, int group_size,
                            float scale2, void* stream);
 
+/* The kernel that ccq_wq_mfma_linear_f32, and the linears above from their
+ * batch sizes on, run for these sizes (formats as above; for tests and
+ * profiles): 0 none (the streaming kernels), 1 up to 64 rows a workgroup, 2 up
+ * to 16 rows with K split over the waves, 3 tiled; tile_rows and tile_cols (may
+ * be NULL): a workgroup's rows and columns. */
+int ccq_wq_linear_kernel(int fmt, int64_t batch, int64_t in_features, int64_t out_features,
+                         int group_size, int* tile_rows, int* tile_cols);
+
+/* The kernel that ccq_int8_linear runs for these sizes (for tests and
+ * profiles): 0 one thread per output, 1 up to 32 rows, 2 and 3 the ring kernel
+ * with 128- and 256-row tiles, 4 the register-staged 128 x 128 tiles, 5 64 x 64
+ * tiles. */
+int ccq_int8_linear_kernel(int64_t M, int64_t K, int64_t N);
+
 /* Bytes of workspace ccq_int8_linear needs for this shape (0: none). */
 size_t ccq_int8_linear_workspace_size(int64_t M, int64_t K, int64_t N);
 
@@ -255,6 +269,11 @@ int64_t ccq_awq_sz_words(int64_t K, int64_t group_size);
  * zero << 16, padding words 0.  Load-time step next to ccq_awq_repack. */
 int ccq_awq_pack_sz(const int32_t* qzeros, const void* scales, int scale_dtype,
                     uint32_t* sz, int64_t K, int64_t N, int64_t group_size, void* stream);
+
+/* The kernel that ccq_w4_gemm runs for these sizes (for tests and profiles): 0
+ * the streaming kernel, 1 the 16-row kernel, 2 the 64-row kernel, 3 the 128-row
+ * grouped kernel; -1 for sizes it refuses. */
+int ccq_w4_gemm_kernel(int64_t M, int64_t K, int64_t N, int64_t group_size);
 
 /* Workspace bytes ccq_w4_gemm takes for these sizes: 0 up to 16 rows.  More
  * than 64 rows of group 128, N % 128 == 0 and K >= 256 need at least the row

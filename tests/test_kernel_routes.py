@@ -1,0 +1,54 @@
+"""Which kernel a linear's sizes run on (the rules are host code: no GPU is
+needed here).  Each row is a side of one of the rules' lines, measured."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+
+STREAM, SKINNY, SLAB, GROUPED = range(4)
+
+
+@pytest.fixture(scope="module")
+def lib(built_lib):
+    from ccut import _lib
+
+    return _lib.lib()
+
+
+@pytest.mark.parametrize("M,K,N,G,kernel", [
+    (1, 4096, 14336, 128, STREAM), (16, 4096, 14336, 128, STREAM), (16, 4096, 14336, 64, SKINNY),
+    (16, 4224, 14336, 128, SKINNY), (64, 4096, 4096, 128, SKINNY), (37, 4096, 14336, 128, SLAB),
+    (2048, 4096, 14336, 64, SLAB), (2048, 4096, 14336, 128, GROUPED),
+    (0, 128, 16, 128, -1), (1, 64, 16, 128, -1), (1, 128, 8, 128, -1), (1, 128, 16, 16, -1),
+])
+def test_awq_linear(lib, M, K, N, G, kernel):
+    assert lib.ccq_w4_gemm_kernel(M, K, N, G) == kernel
+
+
+FP8_ROW, INT8_ROW, MXFP8, MXFP4 = range(4)
+
+
+def wq(lib, fmt, M, K, N, G=32):
+    """(kernel, rows, columns of a workgroup)"""
+    r, c = ctypes.c_int(), ctypes.c_int()
+    return lib.ccq_wq_linear_kernel(fmt, M, K, N, G, ctypes.byref(r), ctypes.byref(c)), r.value, c.value
+
+
+@pytest.mark.parametrize("fmt,M,K,N,route", [
+    (FP8_ROW, 512, 4096, 14336, (3, 128, 256)), (FP8_ROW, 500, 256, 10300, (3, 128, 256)),
+    (FP8_ROW, 260, 256, 7000, (3, 128, 128)), (FP8_ROW, 260, 320, 7000, (3, 128, 128)),
+    (FP8_ROW, 300, 768, 4100, (3, 64, 128)), (FP8_ROW, 16, 4096, 14336, (1, 16, 64)),
+    (FP8_ROW, 16, 4096, 8192, (2, 16, 32)), (MXFP4, 16, 4096, 14336, (2, 16, 64)),
+    (MXFP4, 64, 4096, 14336, (1, 64, 64)), (MXFP4, 12, 4224, 14336, (0, 0, 0)),
+])
+def test_decoded_weight_linear(lib, fmt, M, K, N, route):
+    assert wq(lib, fmt, M, K, N) == route
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (32, 4096, 4096, 1), (1024, 4096, 4096, 2), (4096, 4096, 14336, 3), (1024, 4112, 4096, 4), (40, 20, 100, 0),
+])
+def test_int8_linear(lib, M, K, N, kernel):
+    assert lib.ccq_int8_linear_kernel(M, K, N) == kernel
