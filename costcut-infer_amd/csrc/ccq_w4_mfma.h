@@ -113,9 +113,14 @@ inline bool w4_grouped_shape(int64_t M, int64_t K, int64_t N, int64_t G) {
 // by themselves (M=128 K=2048 N=2048 10.4 us against 22.0, M=65 K=2048 N=9216
 // 15.1 against 24, both the 16-row kernel; M=256 K=4096 N=4096 33 against 17
 // of the slab kernel; past those M=400 K=4096 N=4096 39 against 76 and M=128
-// K=4096 N=14336 40 against 81 and 50).
+// K=4096 N=14336 40 against 81 and 50).  A short K has few waves however many
+// rows there are: past two rounds of 64 x 64 blocks the grouped kernel takes
+// those too (K=512: M=1024 N=2048 13.7 us against 18.6, but M=1024 N=2176 21.6
+// -> 14.1 and M=8192 N=512 31.3 -> 20.5; K=256 the same way, 11.4 against 14.8
+// and 17.0 -> 11.5, 22.7 -> 16.2).
 inline bool w4_grouped_takes(int64_t M, int64_t K, int64_t N, int64_t G) {
-  return w4_grouped_shape(M, K, N, G) && w4_skinny_waves(M, K, N, G) > 2 * 256 * 8 && cdiv(M, 64) * cdiv(N, 64) > 256;
+  const int64_t blocks = cdiv(M, 64) * cdiv(N, 64);
+  return w4_grouped_shape(M, K, N, G) && blocks > 256 && (blocks > 512 || w4_skinny_waves(M, K, N, G) > 2 * 256 * 8);
 }
 bool w4_slab_takes(int64_t M, int64_t K, int64_t N, int64_t G);
 size_t w4_slab_workspace(int64_t M, int64_t K, int64_t N);  // 0 when K is not split

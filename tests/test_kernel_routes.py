@@ -21,6 +21,8 @@ def lib(built_lib):
     (1, 4096, 14336, 128, STREAM), (16, 4096, 14336, 128, STREAM), (16, 4096, 14336, 64, SKINNY),
     (16, 4224, 14336, 128, SKINNY), (64, 4096, 4096, 128, SKINNY), (37, 4096, 14336, 128, SLAB),
     (2048, 4096, 14336, 64, SLAB), (2048, 4096, 14336, 128, GROUPED),
+    # many rows of a short K: two rounds of 64 x 64 blocks, and past those
+    (1024, 512, 2048, 128, SKINNY), (8192, 256, 512, 128, GROUPED), (1024, 512, 2176, 128, GROUPED),
     (0, 128, 16, 128, -1), (1, 64, 16, 128, -1), (1, 128, 8, 128, -1), (1, 128, 16, 16, -1),
 ])
 def test_awq_linear(lib, M, K, N, G, kernel):
