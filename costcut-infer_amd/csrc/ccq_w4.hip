@@ -1217,6 +1217,7 @@ struct W4GP {
   int M, N, K, KT, szw;
   uint32_t nib_mask;           // 0x000F000F (a run-time value, see dq_b3)
   int splits;                  // EPI_STORE: K splits, float32 partials at y + split * M * N (1 = none)
+  int by_rows;                 // EPI_STORE: order of the items (see the kernel)
 };
 
 constexpr int GG_BM = 128;
@@ -1234,7 +1235,10 @@ static_assert(GG_STAGES * GG_STAGE + 3 * GG_RID * 4 + 4 * GG_BM * 4 <= 160 * 102
 
 
 
-template <typename AT, typename ST, int EPI, int CTW>
+// SPLIT (EPI_STORE): K over p.splits workgroups; an instance of its own, since
+// the split's offsets in every k-step cost unsplit calls 2-4% (M=2048 K=4096
+// N=14336 292 -> 287 us, M=4096 N=1152 99.7 -> 97.6 without them).
+template <typename AT, typename ST, int EPI, int CTW, bool SPLIT = false>
 __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   using V = typename Act<AT>::vec;
   constexpr int NQ = EPI == EPI_SILU ? 2 : 1;
@@ -1267,9 +1271,11 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   // order (split, column block, row tile), as many items as the XCD's share of
   // the grid: a column block's weights are read into one L2.  (Row tiles dealt
   // round-robin left a single tile on one XCD: M=128 K=4096 N=14336 531 us;
-  // column blocks innermost, M=2048 305 us against 292.)
+  // column blocks innermost, M=2048 305 us against 292.)  By rows (row tile,
+  // column block) where the activations are by far the larger part: then it
+  // is they that each XCD should read a range of (p.by_rows, ccq_w4_gemm).
   constexpr bool DENSE = EPI == EPI_STORE;
-  const int all = ntiles * nblk * (DENSE ? p.splits : 1);
+  const int all = ntiles * nblk * (SPLIT ? p.splits : 1);
   const int first = DENSE ? xcd * (all >> 3) + min(xcd, all & 7) : 0;
   const int items_x = DENSE ? (all >> 3) + (xcd < (all & 7) ? 1 : 0)
                             : (ntiles > xcd ? (ntiles - xcd + 7) >> 3 : 0) * nblk;
@@ -1284,15 +1290,20 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   const int nmine = items_x / nx + (item_of(items_x / nx) < items_x ? 1 : 0);
   const int per = DENSE ? ntiles * nblk : 1;  // items of one split
   // a split K (then one item per workgroup, see launch_group_gemm) starts at kt0
-  const int split0 = DENSE && p.splits > 1 ? (first + item_of(0)) / per : 0;
-  const int kt0 = DENSE ? (int)((int64_t)p.KT * split0 / p.splits) : 0;
-  const int KT = DENSE ? (int)((int64_t)p.KT * (split0 + 1) / p.splits) - kt0 : p.KT;
+  int split0 = 0, kt0 = 0, KT = p.KT;
+  if constexpr (SPLIT) {  // in SGPRs: they are part of every k-step's addresses
+    split0 = __builtin_amdgcn_readfirstlane((first + item_of(0)) / per);
+    kt0 = __builtin_amdgcn_readfirstlane(p.KT * split0 / p.splits);  // KT < 2^13, splits <= CUs
+    KT = __builtin_amdgcn_readfirstlane(p.KT * (split0 + 1) / p.splits) - kt0;
+  }
   const int total = nmine * KT;  // k-steps of this workgroup
 
   // ---- row ids: rows of item j go to Rid[j % 3], copied (DMA) at the first
   // k-step of item j - 2; Rid[.][GG_BM..] holds the item's expert ----
   auto tile_of = [&](int j) {
-    return DENSE ? (first + item_of(j)) % per % ntiles : xcd + 8 * (item_of(j) / nblk);
+    if constexpr (!DENSE) return xcd + 8 * (item_of(j) / nblk);
+    const int q = SPLIT ? (first + item_of(j)) % per : first + item_of(j);
+    return p.by_rows ? q / nblk : q % ntiles;
   };
   auto fetch_rows = [&](int j) {  // waves 5..7
     if (j >= nmine) return;
@@ -1321,7 +1332,11 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   const bool has_sx = wave == 4 || wave == 5;
   const int ncopy = 4 + BPW + (has_sz ? 1 : 0) + (has_sx ? 1 : 0);
   auto make_plan = [&](int j, Plan& P) {
-    P.nb = DENSE ? (first + item_of(j)) % per / ntiles : item_of(j) % nblk;
+    P.nb = item_of(j) % nblk;
+    if constexpr (DENSE) {
+      const int q = SPLIT ? (first + item_of(j)) % per : first + item_of(j);
+      P.nb = p.by_rows ? q % nblk : q / ntiles;
+    }
     const int* R = Rid[j % 3];
     const int ex = p.tile_expert != nullptr ? __builtin_amdgcn_readfirstlane(R[GG_BM]) : 0;
     // valid rows form a prefix of the tile
@@ -1358,7 +1373,7 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
   const uint32_t lds0 = lds_addr(smem);
   auto issue = [&](const Plan& P, int kt, int slot) {
     const uint32_t st = lds0 + slot * GG_STAGE;
-    if constexpr (DENSE) kt += kt0;
+    if constexpr (SPLIT) kt += kt0;
     const char* xb = reinterpret_cast<const char*>(p.x) + (int64_t)kt * 256;
 #pragma unroll
     for (int i = 0; i < 4; ++i) dma16(xb, P.aoff[i], st + (16 * wave + 4 * i) * 256);
@@ -1564,7 +1579,7 @@ __global__ __launch_bounds__(512) void w4_group_gemm_kernel(const W4GP p) {
             const float fr = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(fs), 0xB1, 0xF, 0xF, false));
             const float lo = odd ? fr : v0, hi = odd ? v1 : fr;  // columns (c & ~1), (c | 1) of the row
             if (row < P.nvalid) {
-              const int64_t o = (int64_t)R[row] * p.ldy + col2 + c * 32 + (DENSE ? (int64_t)split0 * p.M * p.N : 0);
+              const int64_t o = (int64_t)R[row] * p.ldy + col2 + c * 32 + (SPLIT ? (int64_t)split0 * p.M * p.N : 0);
               if (p.y_dtype == CCQ_F32)
                 *reinterpret_cast<f32x2*>(reinterpret_cast<float*>(p.y) + o) = f32x2{lo, hi};
               else if (p.y_dtype == CCQ_BF16)
@@ -1736,7 +1751,11 @@ static int launch_group_gemm(const W4GP& p, int x_bf16, int s_bf16, int64_t tile
   const dim3 grid((unsigned)(EPI == EPI_STORE && items < 8 ? 8 : (items < cus ? items : cus))), block(512);
 #define CCQ_LAUNCH_GG(AT, ST)                                                                  \
   do {                                                                                         \
-    if (wgn == 256)                                                                            \
+    if (EPI == EPI_STORE && p.splits > 1 && wgn == 256)                                        \
+      launch((w4_group_gemm_kernel<AT, ST, EPI, (EPI == EPI_SILU ? 2 : 4), EPI == EPI_STORE>), grid, block, 0, st, p); \
+    else if (EPI == EPI_STORE && p.splits > 1)                                                 \
+      launch((w4_group_gemm_kernel<AT, ST, EPI, 2, EPI == EPI_STORE>), grid, block, 0, st, p); \
+    else if (wgn == 256)                                                                       \
       launch((w4_group_gemm_kernel<AT, ST, EPI, (EPI == EPI_SILU ? 2 : 4)>), grid, \
                          block, 0, st, p);                                                     \
     else                                                                                       \
@@ -1943,6 +1962,11 @@ extern "C" int ccq_w4_gemm(const void* x, int x_dtype, const int32_t* w_tiled, c
     g.szw = (int)sz_words_per_column(K, group_size);
     g.nib_mask = 0x000F000Fu;
     g.splits = workspace_bytes >= base + group_partials(M, K, N) && aligned(y, 16) ? group_splits(M, K, N) : 1;
+    // items by rows where the activations are 7 and more times the weight
+    // (M=8192 K=4096 N=2176 250.7 -> 241.2 us, N=1152 156 -> 150; below or with
+    // a short K the same or worse: M=2500 N=3072 83.5 against 85.8, K=256
+    // M=8192 N=2176 36.2 against 38.0)
+    g.by_rows = g.splits == 1 && K >= 1024 && 4 * M > 7 * N;
     if (g.splits > 1) {
       g.y = (char*)workspace + base;
       g.y_dtype = CCQ_F32;
