@@ -393,9 +393,40 @@ SlabPlan plan_slab(int64_t M, int64_t K, int64_t N) {
 // Of the grouped kernel's shapes it takes those of one round of its blocks
 // (M=128 K=4096 N=4096 22.6 us of the 16-row kernel -> 16.4, M=130 K=7168
 // N=2432 34.5 -> 18.4; two rounds: M=65 K=2048 N=9216 15.1 against 20.2).
+//
+// What the count of waves does not see, shapes where the 16-row kernel stays
+// (us of it against this kernel; N % 32 != 0 is left out of most, its
+// workgroups are narrower and slower there):
+//  * a second round of 64 x 64 blocks that is nearly empty: up to 12 k-tiles for
+//    groups 32 and 64 (G=32 M=128 K=1536 N=8256 26.9 against 28.4, M=96 21.7
+//    against 23.5) and for up to 64 rows (G=128 M=64 K=1024 N=18432 15.2
+//    against 16.8), and for 65 to 80 rows, which are 48-row blocks, also past
+//    those (G=128 M=65 K=2048 N=8224 17.9 against 20.0, G=64 K=1664 16.7 against
+//    21.4);
+//  * groups 32 and 64 of one or two k-tiles (G=64 M=2048 K=256 N=4096 28.9 against
+//    36.4; G=32 only for few rows, M=65 N=14336 7.9 against 10.0);
+//  * group 64 with K of 768 and 1024, where two waves of the 16-row kernel share a
+//    workgroup's columns and N % 128 == 0 keeps them on one XCD (M=2048 K=1024
+//    N=4096 64.2 against 69.1; K=512, 896 and 1536 are this kernel's);
+//  * groups 32 and 64 on few blocks whose K is not split (under 32 k-tiles) or
+//    just split in two: one CU per block against up to three workgroups on each
+//    (G=32 M=128 K=3072 N=2048 15.7 against 24.9, M=64 N=4096 16.0 against 25.0;
+//    G=64 M=512 N=1024 18.7 against 20.1).
+static bool w4_skinny_stays(int64_t M, int64_t K, int64_t N, int64_t G) {
+  const int64_t KT = K / 128, blocks = cdiv(M, 64) * cdiv(N, 64);
+  const bool wide = N % 32 == 0, second = blocks > 256 && blocks <= 320;
+  if (wide && second && M > 64 && M <= 80 && (G == 64 || KT <= 16)) return true;
+  if (wide && second && M > 32 && KT >= 6 && KT <= 12 && (G < 128 || M <= 64)) return true;
+  if (G == 128) return false;
+  if (wide && KT <= 2 && (G == 64 || M <= 80)) return true;
+  if (G == 64) return N % 128 == 0 && (KT == 6 || KT == 8 || (blocks <= 128 && KT < 32 && M > 128));
+  return blocks <= 128 && KT <= 32 && M > 32 && cdiv(M, 16) * cdiv(N, 32) * KT <= (KT < 32 ? 18432 : 16384);
+}
+
 bool w4_slab_takes(int64_t M, int64_t K, int64_t N, int64_t G) {
   const int64_t blocks = cdiv(M, 64) * cdiv(N, 64);
   return M > 16 && w4_skinny_waves(M, K, N, G) > 256 * 8 && (!w4_grouped_shape(M, K, N, G) || blocks <= 256) &&
+         !w4_skinny_stays(M, K, N, G) &&
          64 * K * 2 < (1LL << 32) && N * sz_words_per_column(K, G) * 4 < (1LL << 32) && blocks <= 0x7fffffff;
 }
 

@@ -23,6 +23,12 @@ def lib(built_lib):
     (2048, 4096, 14336, 64, SLAB), (2048, 4096, 14336, 128, GROUPED),
     # many rows of a short K: two rounds of 64 x 64 blocks, and past those
     (1024, 512, 2048, 128, SKINNY), (8192, 256, 512, 128, GROUPED), (1024, 512, 2176, 128, GROUPED),
+    # where the 64-row kernel would be slower than the 16-row one, and just past
+    (65, 2048, 8224, 128, SKINNY), (65, 2176, 8224, 128, SLAB), (96, 2048, 8224, 128, SLAB),
+    (128, 1536, 8256, 32, SKINNY), (128, 1664, 8256, 32, SLAB), (128, 640, 8256, 32, SLAB),
+    (2048, 256, 4096, 64, SKINNY), (2048, 384, 4096, 64, SLAB), (65, 256, 14336, 32, SKINNY), (96, 256, 14336, 32, SLAB),
+    (2048, 1024, 4096, 64, SKINNY), (2048, 1152, 4096, 64, SLAB), (2048, 512, 4096, 64, SLAB), (2048, 1024, 4160, 64, SLAB),
+    (128, 3072, 2048, 32, SKINNY), (64, 3072, 4096, 32, SKINNY), (64, 3072, 8192, 32, SLAB), (512, 3072, 1024, 64, SKINNY),
     (0, 128, 16, 128, -1), (1, 64, 16, 128, -1), (1, 128, 8, 128, -1), (1, 128, 16, 16, -1),
 ])
 def test_awq_linear(lib, M, K, N, G, kernel):
