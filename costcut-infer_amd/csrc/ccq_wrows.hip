@@ -174,11 +174,23 @@ int wq_rows_route(int fmt, bool g16, int64_t M, int64_t K, int64_t N) {
   // With 64 columns the 64-row kernel keeps the one-byte formats: K=4096 N=14336
   // M=16, weights from HBM (12 sets in turn), fp8 20.7 us against 22.9 and MXFP8
   // 27.0 against 28.2 (from the Infinity Cache 20.0 against 18.0 and 26.1
-  // against 23.8); MXFP4 20.7 -> 17.4 at M=1 and 23.5 -> 18.8 at M=16.  And short
-  // K, where a wave has no third k-tile to load ahead (MXFP4 K=1024 N=12000 9.9
-  // against 10.8, K=2048 N=9000 13.0 -> 11.5).  32 columns: K=6144 N=8192 M=16
-  // fp8 27.4 -> 14.9, MXFP4 29.8 -> 14.5.
-  if (nb == 4 && (fmt != WQ_MXFP4 || K < 2048)) return 0;
+  // against 23.8).  MXFP4: 19.7 -> 17.5 at M=1 and 22.1 -> 19.7 at M=16, but not
+  // where each wave has three k-tiles, which its loop takes in pairs (K=3072
+  // M=1 15.7 against 17.1), nor with 16-element groups unless the waves have
+  // two or four k-tiles each, or more than that (K=2304 M=1 13.6 against 16.8,
+  // K=4352 22.3 against 24.4; K=4096 M=16 23.4 -> 22.0, K=5120 31.2 -> 28.0).
+  if (nb == 4) return fmt == WQ_MXFP4 && (g16 ? K % 2048 == 0 || K >= 5120 : K >= 2048 && K != 3072) ? nb : 0;
+  // A short K, where a wave has no third k-tile to load ahead.  32 columns
+  // (N=8192 M=16): fp8 K=1536 8.9 against 9.5, K=2048 10.7 -> 9.6; MXFP8 K=1280 9.1
+  // against 10.0, 16-element groups K=512 5.8 against 7.1; MXFP4 K=256 3.9 against
+  // 4.2, K=512 5.1 -> 4.9, 16-element groups K=512 5.8 against 6.4, K=768 7.1 ->
+  // 7.0.  16 columns: the MX formats with K=256 (16-element groups, M=1 N=33 2.8
+  // against 3.5).
+  const int64_t shortest = fmt < WQ_MXFP8 ? (nb == 2 ? 2048 : 256)
+                           : nb == 1      ? 512
+                           : fmt == WQ_MXFP8 ? 1536
+                                             : (g16 ? 768 : 512);
+  if (K < shortest) return 0;
   return nb;
 }
 

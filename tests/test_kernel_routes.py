@@ -49,10 +49,24 @@ def wq(lib, fmt, M, K, N, G=32):
     (FP8_ROW, 260, 256, 7000, (3, 128, 128)), (FP8_ROW, 260, 320, 7000, (3, 128, 128)),
     (FP8_ROW, 300, 768, 4100, (3, 64, 128)), (FP8_ROW, 16, 4096, 14336, (1, 16, 64)),
     (FP8_ROW, 16, 4096, 8192, (2, 16, 32)), (MXFP4, 16, 4096, 14336, (2, 16, 64)),
+    # a short K stays on the 64-row kernel, by columns of a workgroup
+    (FP8_ROW, 16, 256, 4096, (2, 16, 16)), (FP8_ROW, 16, 1792, 4100, (1, 16, 64)), (INT8_ROW, 4, 1024, 8192, (1, 16, 64)),
+    (FP8_ROW, 16, 2048, 8192, (2, 16, 32)), (MXFP8, 1, 256, 33, (1, 16, 64)), (MXFP8, 1, 512, 33, (2, 16, 16)),
+    (MXFP8, 16, 1280, 8192, (1, 16, 64)), (MXFP8, 16, 1536, 8192, (2, 16, 32)), (MXFP4, 16, 256, 8192, (1, 16, 64)),
+    (MXFP4, 16, 512, 8192, (2, 16, 32)), (MXFP4, 1, 3072, 14336, (1, 16, 64)), (MXFP4, 1, 3328, 14336, (2, 16, 64)),
     (MXFP4, 64, 4096, 14336, (1, 64, 64)), (MXFP4, 12, 4224, 14336, (0, 0, 0)),
 ])
 def test_decoded_weight_linear(lib, fmt, M, K, N, route):
     assert wq(lib, fmt, M, K, N) == route
+
+
+@pytest.mark.parametrize("fmt,M,K,N,route", [
+    (MXFP4, 16, 512, 8192, (1, 16, 64)), (MXFP4, 16, 768, 8192, (2, 16, 32)), (MXFP4, 16, 2048, 14336, (2, 16, 64)),
+    (MXFP4, 16, 2304, 14336, (1, 16, 64)), (MXFP4, 16, 4096, 14336, (2, 16, 64)), (MXFP4, 16, 4352, 14336, (1, 16, 64)),
+    (MXFP4, 16, 5120, 14336, (2, 16, 64)), (MXFP8, 16, 512, 8192, (1, 16, 64)),
+])
+def test_decoded_weight_linear_groups_of_16(lib, fmt, M, K, N, route):
+    assert wq(lib, fmt, M, K, N, 16) == route
 
 
 @pytest.mark.parametrize("M,K,N,kernel", [
