@@ -305,12 +305,23 @@ bool wq_tile_route(int fmt, int64_t M, int64_t K, int64_t N, int& bm, int& bn) {
     // the CUs (fp8 M=512 K=N=2048 26 us against 28; MXFP4 25 against 33); past
     // that fp8 K=4096 N=14336 M=65 79 -> 47 us, M=128 97 -> 49, M=512 332 -> 129
     if (M <= 64 || cdiv(M, 64) * cdiv(N, 64) <= 256) return false;
-  } else if (M <= 12 || M * N < (fmt >= WQ_MXFP8 ? 1 << 17 : 3 << 16)) {
+  } else {
     // a workgroup takes about 1 us per chunk however few there are, the
     // streaming kernels a time in proportion to M N (K=2176 N=4001 M=33: int8
     // 36.6 us against 37.6, MXFP4 62 against 44; K=4224 N=14336: int8 M=10 52
-    // against 68, M=16 79 against 68, M=64 310 -> 70, M=512 2506 -> 241)
-    return false;
+    // against 68, M=16 79 against 68, M=64 310 -> 70, M=512 2506 -> 241), and
+    // with a longer K they do better (M=48 N=4096, M N = 3 << 16: int8 K=1600 33.3
+    // -> 32.0, K=6208 90 against 113; M=32 N=4096, 1 << 17: MXFP8 K=1088 26.0 ->
+    // 21.9, K=2176 35.4 against 40.6, K=4224 55.6 against 76.0)
+    int64_t least = 3 << 16;  // M N from which the tiles are faster
+    if (fmt == WQ_MXFP4) {
+      least = 1 << 17;
+    } else if (fmt == WQ_MXFP8) {
+      least = K <= 1344 ? 1 << 17 : (K <= 2432 ? 9 << 14 : (3 << 16) + 1);
+    } else if (K >= 2048) {
+      least = fmt == WQ_INT8_ROW && K >= 4096 ? 7 << 15 : (3 << 16) + 1;
+    }
+    if (M <= 12 || M * N < least) return false;
   }
   // the largest tile that still gives most CUs one
   bm = 128;

@@ -54,6 +54,11 @@ def wq(lib, fmt, M, K, N, G=32):
     (FP8_ROW, 16, 2048, 8192, (2, 16, 32)), (MXFP8, 1, 256, 33, (1, 16, 64)), (MXFP8, 1, 512, 33, (2, 16, 16)),
     (MXFP8, 16, 1280, 8192, (1, 16, 64)), (MXFP8, 16, 1536, 8192, (2, 16, 32)), (MXFP4, 16, 256, 8192, (1, 16, 64)),
     (MXFP4, 16, 512, 8192, (2, 16, 32)), (MXFP4, 1, 3072, 14336, (1, 16, 64)), (MXFP4, 1, 3328, 14336, (2, 16, 64)),
+    # in_features % 256 != 0: rows times columns from which the tiles are faster
+    (INT8_ROW, 48, 1600, 4096, (3, 64, 128)), (INT8_ROW, 48, 2112, 4096, (0, 0, 0)), (INT8_ROW, 49, 2112, 4096, (3, 64, 128)),
+    (INT8_ROW, 51, 4224, 4096, (0, 0, 0)), (INT8_ROW, 56, 4224, 4096, (3, 64, 128)), (FP8_ROW, 49, 4224, 4096, (3, 64, 128)),
+    (MXFP8, 32, 1088, 4096, (3, 64, 128)), (MXFP8, 32, 2176, 4096, (0, 0, 0)), (MXFP8, 36, 2176, 4096, (3, 64, 128)),
+    (MXFP8, 48, 4224, 4096, (0, 0, 0)), (MXFP8, 49, 4224, 4096, (3, 64, 128)), (MXFP4, 32, 4224, 4096, (3, 64, 128)),
     (MXFP4, 64, 4096, 14336, (1, 64, 64)), (MXFP4, 12, 4224, 14336, (0, 0, 0)),
 ])
 def test_decoded_weight_linear(lib, fmt, M, K, N, route):
