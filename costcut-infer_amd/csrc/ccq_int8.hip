@@ -583,10 +583,16 @@ bool int8_big(int64_t M, int64_t K, int64_t N) {
   return M > I8_SKINNY_M && M * K < ((int64_t)1 << 31) && N * K < ((int64_t)1 << 31);
 }
 
-// the ring kernel (K % 128 == 0), and its tile height: 256 rows where those
-// tiles still cover the CUs
+// the ring kernel (K % 128 == 0), and its tile height: 256 rows (4 KiB of operand
+// reads for 4 MFMAs instead of 3 for 2) where those tiles take well fewer rounds
+// of the CUs than 128-row ones (M=4096 K=1024 N=5120, 3 rounds against 5: 63 us
+// against 69; 2 against 3 is a loss: M=257 K=512 N=28672 31.6 against 26.5, M=1536
+// K=4096 N=8192 82.3 against 78.7)
 bool int8_ring(int64_t M, int64_t K, int64_t N) { return int8_big(M, K, N) && K % 128 == 0; }
-int int8_ring_rt(int64_t M, int64_t N) { return cdiv(M, 256) * cdiv(N, 128) >= 256 ? 2 : 1; }
+int int8_ring_rt(int64_t M, int64_t N) {
+  const int64_t nt = cdiv(N, 128), tall = cdiv(M, 256) * nt;
+  return tall >= 256 && 5 * cdiv(cdiv(M, 128) * nt, 256) >= 8 * cdiv(tall, 256) ? 2 : 1;
+}
 
 int int8_splits(int64_t M, int64_t K, int64_t N) {
   if (K == 0 || K % 16 != 0) return 1;

@@ -76,6 +76,8 @@ def test_decoded_weight_linear_groups_of_16(lib, fmt, M, K, N, route):
 
 @pytest.mark.parametrize("M,K,N,kernel", [
     (32, 4096, 4096, 1), (1024, 4096, 4096, 2), (4096, 4096, 14336, 3), (1024, 4112, 4096, 4), (40, 20, 100, 0),
+    # rounds of the CUs with 256- and with 128-row tiles: 3 and 5, 2 and 3, 1 and 2
+    (4096, 1024, 5120, 3), (257, 512, 28672, 2), (1536, 4096, 8192, 2), (260, 1280, 16500, 2), (260, 1280, 16300, 3),
 ])
 def test_int8_linear(lib, M, K, N, kernel):
     assert lib.ccq_int8_linear_kernel(M, K, N) == kernel
