@@ -25,8 +25,9 @@
 // Weights are exact in bf16 except MXFP8 codes under the E8M0 bytes 1 and 2
 // (scales 2^-126 and 2^-125), which reach below bf16's smallest step 2^-133.
 // With three parts (the float32 kernels took those shapes) a workgroup that
-// meets such a byte runs its chunks again with what the rounding left over,
-// times 2^64 (wq_tiny8); others pay an OR per scale byte.
+// meets such a byte starts over: once with bf16 weights that are zero only
+// where the weight is, once with 2^64 times what those leave (wq_tiny8).  The
+// others pay an OR per scale byte.
 //
 // Sums: the MFMAs add up 128 k, and these spans are added on the VALU: K / 16
 // dependent roundings in one chain would cost more than the parts do (K=2176:
@@ -41,9 +42,9 @@ namespace {
 
 constexpr int WT_KC = 64;
 
-// 8 floats -> NSP bf16 pieces of 16 bytes (FIN, three parts: Inf and NaN -> 0)
-template <int NSP, bool FIN = false>
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[NSP]) {
+// 8 floats -> NSP bf16 pieces of 16 bytes (fin_only, three parts: Inf and NaN -> 0)
+template <int NSP>
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[NSP], bool fin_only) {
   if constexpr (NSP == 2) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -60,7 +61,7 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[NSP]) {
       const float r = fin ? v[e] - __uint_as_float(u & 0xffff0000u) : 0.f;
       const uint32_t ur = __float_as_uint(r);
       // a NaN stays one when its low bits go
-      p[0][e] = FIN && !fin ? 0u : (!fin && (u & 0x007fffffu) ? u | 0x00400000u : u);
+      p[0][e] = fin_only && !fin ? 0u : (!fin && (u & 0x007fffffu) ? u | 0x00400000u : u);
       p[1][e] = ur;
       p[2][e] = __float_as_uint(r - __uint_as_float(ur & 0xffff0000u));
     }
@@ -72,10 +73,9 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[NSP]) {
 }
 
 // Eight MXFP8 weights under the scale byte 1 or 2: rounded to bf16, but never to
-// zero (Inf times a weight that is not zero is no NaN), or (LEFT) 2^64 times
+// zero (Inf times a weight that is not zero is no NaN), or (left) 2^64 times
 // what that leaves, at most three steps of 2^-135: exact.
-template <bool LEFT>
-__device__ __forceinline__ bf16x8 wq_tiny8(uint32_t w0, uint32_t w1, uint32_t e) {
+__device__ __forceinline__ bf16x8 wq_tiny8(uint32_t w0, uint32_t w1, uint32_t e, bool left) {
   const float s = e8m0_to_f32(e);
   float o[8];
 #pragma unroll
@@ -83,7 +83,7 @@ __device__ __forceinline__ bf16x8 wq_tiny8(uint32_t w0, uint32_t w1, uint32_t e)
     const float v = fp8_e4m3_to_f32(((j < 4 ? w0 : w1) >> (8 * (j & 3))) & 0xFFu) * s;
     uint32_t h = f32_to_bf16_bits(v);
     if (!(h & 0x7FFFu) && v != 0.f) h |= 1u;
-    o[j] = LEFT ? (v - bf16_bits_to_f32(h)) * 0x1p64f : bf16_bits_to_f32(h);
+    o[j] = left ? (v - bf16_bits_to_f32(h)) * 0x1p64f : bf16_bits_to_f32(h);
   }
   return pack_bf16x8(o);
 }
@@ -157,14 +157,14 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
     }
   };
   bool tiny = false;  // a scale byte 1 or 2 in this thread's weights
-  auto store = [&](int buf, auto left_c) {
-    constexpr bool LEFT = decltype(left_c)::value;
+  auto store = [&](int buf, auto exact_c, bool left) {
+    constexpr bool EXACT = decltype(exact_c)::value;
     char* S = smem + buf * BUF;
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
       const float v[8] = {xr[i][0].x, xr[i][0].y, xr[i][0].z, xr[i][0].w, xr[i][1].x, xr[i][1].y, xr[i][1].z, xr[i][1].w};
       u32x4 o[NSP];
-      split8<NSP, LEFT>(v, o);
+      split8<NSP>(v, o, EXACT && left);
 #pragma unroll
       for (int q = 0; q < NSP; ++q) *reinterpret_cast<u32x4*>(S + q * A_PART + xd[i]) = o[q];
     }
@@ -174,13 +174,16 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
       const uint32_t e = Tr::MX ? sr[NSC == 2 ? j * 8 / G : 0] & 255u : 0u;
       if constexpr (FMT == WQ_MXFP4)
         b = mx4_word_bf16(wr[j], mx4_lut(e));
-      else if (TINY && e - 1u < 2u)
-        b = wq_tiny8<LEFT>(wr[2 * j], wr[2 * j + 1], e);
-      else if constexpr (LEFT)
-        b = bf16x8{};
       else
         b = wq_decode8<FMT>(wr[2 * j], wr[2 * j + 1], Tr::MX ? e8m0_to_f32(e) : 1.f);
-      if constexpr (TINY) tiny |= e - 1u < 2u;
+      if constexpr (EXACT) {
+        if (e - 1u < 2u)
+          b = wq_tiny8(wr[2 * j], wr[2 * j + 1], e, left);
+        else if (left)
+          b = bf16x8{};
+      } else if constexpr (TINY) {
+        tiny |= e - 1u < 2u;
+      }
       const int piece = wk / 8 + j;
       *reinterpret_cast<bf16x8*>(S + A_BYTES + wrow * 128 + ((piece ^ ((wrow >> 1) & 7)) * 16)) = b;
     }
@@ -238,25 +241,33 @@ __global__ __launch_bounds__(512, 2) void wq_tile_kernel(const WqP p) {
     }
   };
 
-  auto chunks = [&](auto left_c, auto&& span_done) {
+  auto chunks = [&](auto exact_c, bool left, auto&& span_done) {
     load(0);
-    store(0, left_c);
+    store(0, exact_c, left);
     lds_barrier();
     for (int c = 0; c < nch; ++c) {
       if (c + 1 < nch) load(c + 1);
       multiply(c & 1);
       if ((c & 1) || c + 1 == nch) span_done();
-      if (c + 1 < nch) store((c + 1) & 1, left_c);  // last read in chunk c - 1, before the last barrier
+      if (c + 1 < nch) store((c + 1) & 1, exact_c, left);  // last read in chunk c - 1, before the last barrier
       lds_barrier();
     }
   };
-  chunks(std::false_type{}, [&] { fold(acc, t, 1.f); });
+  chunks(std::false_type{}, false, [&] { fold(acc, t, 1.f); });
 
   if constexpr (NSP == 3) fold(acc, small, 1.f);
   if constexpr (TINY) {
     if (__syncthreads_or(tiny)) {
-      chunks(std::true_type{}, [&] { fold(small, t, 1.f); });
-      fold(acc, small, 0x1p-64f);
+      for (int left = 0; left < 2; ++left) {
+        if (!left) {
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) acc[r][c] = f32x16{};
+        }
+        chunks(std::true_type{}, left, [&] { fold(left ? small : acc, t, 1.f); });
+        fold(acc, small, left ? 0x1p-64f : 1.f);
+      }
     }
   }
 
