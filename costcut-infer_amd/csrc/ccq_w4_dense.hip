@@ -410,8 +410,10 @@ SlabPlan plan_slab(int64_t M, int64_t K, int64_t N) {
 //    N=4096 64.2 against 69.1; K=512, 896 and 1536 are this kernel's);
 //  * groups 32 and 64 on few blocks whose K is not split (under 32 k-tiles) or
 //    just split in two: one CU per block against up to three workgroups on each
-//    (G=32 M=128 K=3072 N=2048 15.7 against 24.9, M=64 N=4096 16.0 against 25.0;
-//    G=64 M=512 N=1024 18.7 against 20.1).
+//    (G=32 M=128 K=3072 N=2048 15.7 against 24.9, M=64 N=4096 16.0 against 25.0,
+//    768 workgroups M=768 N=512 22.6 against 25.0, but M=121 K=2176 N=4096 23.6 ->
+//    20.0; 48-row blocks take less, M=139 K=2816 N=2112 22.3 -> 19.1; G=64 M=512
+//    K=3072 N=1024 18.7 against 20.1).
 static bool w4_skinny_stays(int64_t M, int64_t K, int64_t N, int64_t G) {
   const int64_t KT = K / 128, blocks = cdiv(M, 64) * cdiv(N, 64);
   const bool wide = N % 32 == 0, second = blocks > 256 && blocks <= 320;
@@ -420,7 +422,9 @@ static bool w4_skinny_stays(int64_t M, int64_t K, int64_t N, int64_t G) {
   if (G == 128) return false;
   if (wide && KT <= 2 && (G == 64 || M <= 80)) return true;
   if (G == 64) return N % 128 == 0 && (KT == 6 || KT == 8 || (blocks <= 128 && KT < 32 && M > 128));
-  return blocks <= 128 && KT <= 32 && M > 32 && cdiv(M, 16) * cdiv(N, 32) * KT <= (KT < 32 ? 18432 : 16384);
+  const int64_t wgs = cdiv(M, 16) * cdiv(N, 32), mt = cdiv(cdiv(M, 16), cdiv(M, 64));
+  const int64_t most = KT <= 16 ? 18432 / KT : (KT < 28 ? 768 : (KT < 32 ? 680 : 512));  // workgroups of its rounds
+  return blocks <= 128 && KT <= 32 && M > 32 && wgs <= (mt == 3 ? most * 7 / 10 : most);
 }
 
 bool w4_slab_takes(int64_t M, int64_t K, int64_t N, int64_t G) {

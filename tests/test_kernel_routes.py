@@ -29,6 +29,7 @@ def lib(built_lib):
     (2048, 256, 4096, 64, SKINNY), (2048, 384, 4096, 64, SLAB), (65, 256, 14336, 32, SKINNY), (96, 256, 14336, 32, SLAB),
     (2048, 1024, 4096, 64, SKINNY), (2048, 1152, 4096, 64, SLAB), (2048, 512, 4096, 64, SLAB), (2048, 1024, 4160, 64, SLAB),
     (128, 3072, 2048, 32, SKINNY), (64, 3072, 4096, 32, SKINNY), (64, 3072, 8192, 32, SLAB), (512, 3072, 1024, 64, SKINNY),
+    (768, 3072, 512, 32, SKINNY), (121, 2176, 4096, 32, SLAB), (139, 2816, 2112, 32, SLAB),
     (0, 128, 16, 128, -1), (1, 64, 16, 128, -1), (1, 128, 8, 128, -1), (1, 128, 16, 16, -1),
 ])
 def test_awq_linear(lib, M, K, N, G, kernel):
