@@ -66,6 +66,16 @@ def test_dequant_bitexact(gpu, G, sdt):
     assert np.array_equal(W.view(np.uint32), ref.view(np.uint32))
 
 
+STREAM, SKINNY, SLAB, GROUPED = range(4)
+
+
+def _kernel(M, K, N, G):
+    """The kernel that these sizes run on."""
+    from ccut._lib import lib
+
+    return lib().ccq_w4_gemm_kernel(M, K, N, G)
+
+
 def _gemm_case(gpu, M, K, N, G, xdt, ydt, seed):
     from ccut.quant import awq
 
@@ -88,17 +98,18 @@ def test_gemm_parity_m_sweep(gpu, M, xdt):
 
 @pytest.mark.parametrize("M", [65, 128, 200, 513])
 @pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
-def test_gemm_prefill_grouped_kernel(gpu, M, xdt):
-    """M > 64 with group 128 and N % 128 == 0 runs the tiled prefill kernel
-    (64/128-row tiles, activations staged in LDS)."""
+def test_gemm_prefill_few_columns(gpu, M, xdt):
+    """More than 64 rows on few columns: the 16-row kernel."""
+    assert _kernel(M, 768, 384, 128) == SKINNY
     assert _gemm_case(gpu, M, 768, 384, 128, xdt, torch.float32, seed=M) <= TIGHT
     assert _gemm_case(gpu, M, 768, 384, 128, xdt, xdt, seed=M + 1) <= TOL
 
 
 @pytest.mark.parametrize("M,K,N", [(200, 384, 512), (130, 256, 256), (300, 640, 384), (97, 1024, 768)])
-def test_gemm_prefill_grouped_shapes(gpu, M, K, N):
-    """Grouped kernel with 256-column blocks (N % 256 == 0) and 128-column
-    blocks, odd and even numbers of k-tiles."""
+def test_gemm_prefill_small_products(gpu, M, K, N):
+    """Products of more than 64 rows that the 16-row kernel does in two rounds of
+    the CUs, odd and even numbers of k-tiles."""
+    assert _kernel(M, K, N, 128) == SKINNY
     assert _gemm_case(gpu, M, K, N, 128, torch.bfloat16, torch.float32, seed=M + K) <= TIGHT
     assert _gemm_case(gpu, M, K, N, 128, torch.float16, torch.float32, seed=M + N) <= TIGHT
 
@@ -110,22 +121,26 @@ def test_gemm_parity_groups(gpu, G):
 
 @pytest.mark.parametrize("M,K,N,G", [(17, 4096, 9232, 128), (33, 4480, 6160, 128), (49, 1152, 11024, 128),
                                      (64, 4224, 5200, 64), (40, 3200, 7184, 64), (32, 2176, 9232, 32),
-                                     (48, 4480, 5136, 32), (64, 3200, 4112, 32)])
+                                     (48, 4480, 5136, 32), (64, 3200, 8208, 32)])
 def test_gemm_slab_kernel(gpu, M, K, N, G):
     """17 to 64 rows on enough columns that the 16-row kernel would need a
     second round of workgroups: 2, 3 and 4 row tiles, part-filled last rows and
     columns, k-tile counts that are no multiple of a step's, K split in two
     (K=4480 with few columns) and without the workspace of a split."""
+    assert _kernel(M, K, N, G) == SLAB
     assert _gemm_case(gpu, M, K, N, G, torch.bfloat16, torch.float32, seed=M) <= TIGHT
     assert _gemm_case(gpu, M, K, N, G, torch.float16, torch.float16, seed=M + 1) <= TOL
 
 
 @pytest.mark.parametrize("M,K,N", [(65, 4096, 9216), (260, 3840, 3712), (257, 3712, 4352), (513, 1152, 2944),
-                                   (1150, 1152, 1152), (2100, 640, 2176)])
+                                   (1900, 1152, 1152), (2100, 640, 2176), (2100, 640, 4352), (1100, 256, 8448),
+                                   (1100, 384, 8448), (4200, 1024, 1152), (4200, 1024, 2048)])
 def test_gemm_grouped_dense_schedule(gpu, M, K, N):
     """The 128-row kernel on few and many row tiles: K split over 9, 10, 13 or
     more workgroups per XCD share (odd k-tile counts, part-filled last tiles),
-    unsplit with several items per workgroup."""
+    unsplit with several items per workgroup of 128 and of 256 columns, two and
+    three k-tiles, items by column blocks and (4200 rows) by row tiles."""
+    assert _kernel(M, K, N, 128) == GROUPED
     assert _gemm_case(gpu, M, K, N, 128, torch.bfloat16, torch.float32, seed=M) <= TIGHT
     assert _gemm_case(gpu, M, K, N, 128, torch.float16, torch.float16, seed=M + 1) <= TOL
 
@@ -135,7 +150,32 @@ def test_gemm_grouped_dense_schedule(gpu, M, K, N):
 def test_gemm_slab_kernel_row_blocks(gpu, M, K, N, G):
     """More than 64 rows: shapes the 128-row kernel does not take, and those of
     its shapes whose 64 x 64 blocks are one round of the CUs."""
+    assert _kernel(M, K, N, G) == SLAB
     assert _gemm_case(gpu, M, K, N, G, torch.bfloat16, torch.float32, seed=M) <= TIGHT
+
+
+@pytest.mark.parametrize("M,K,N,G,kernel", [(33, 4480, 6160, 128, SLAB), (64, 4224, 5200, 64, SLAB),
+                                            (65, 1152, 11024, 64, SLAB), (257, 3712, 4352, 128, GROUPED),
+                                            (257, 3712, 3968, 128, GROUPED), (2100, 640, 2176, 128, GROUPED),
+                                            (2100, 640, 4352, 128, GROUPED)])
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+def test_gemm_bf16_scales_and_outputs(gpu, M, K, N, G, kernel, xdt):
+    """Bfloat16 scales, and bfloat16 outputs, of the 64- and the 128-row kernel
+    (128- and 256-column blocks), K split and not: float32 outputs as tight as
+    with float16 scales, bfloat16 ones within their rounding of those."""
+    from ccut.quant import awq
+
+    assert _kernel(M, K, N, G) == kernel
+    qw, qz, s = _make(K, N, G, M, scale_dtype=None)
+    sb = torch.from_numpy(s).to(torch.bfloat16)
+    w = awq.prepare(torch.from_numpy(qw).to(gpu), torch.from_numpy(qz).to(gpu), sb.to(gpu), G)
+    assert w.scale_dtype == torch.bfloat16
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(M)).to(xdt)
+    y = awq.gemm(x.to(gpu), w, out_dtype=torch.float32)
+    ref = oawq.linear(x.float().numpy(), qw, qz, sb.float().numpy(), G)
+    assert np.abs(y.cpu().numpy() - ref).max() <= TIGHT * np.abs(ref).max()
+    for ydt in (torch.bfloat16, torch.float16):
+        assert torch.equal(awq.gemm(x.to(gpu), w, out_dtype=ydt), y.to(ydt))  # one rounding of the same sums
 
 
 def test_gemm_split_k_on_two_streams(gpu):

@@ -145,15 +145,18 @@ def test_w8a8_fused_matches_two_kernels(gpu, M, K, N):
         assert _same(y.cpu().numpy(), y2.cpu().numpy())
 
 
-@pytest.mark.parametrize("M,K,N", [(33, 128, 1), (129, 384, 257), (257, 4096, 33), (40, 1664, 130), (260, 256, 16500),
-                                   (128, 896, 512)])
-def test_int8_ring_kernel_exact(gpu, M, K, N):
-    """The prefill kernel of K % 128 == 0: one chunk, fewer chunks than its
-    ring, K split, part-filled rows and columns, and the 256-row tiles (260 x
-    16500).  Sums are whole numbers below 2^53, exact in float64, so y must be
-    bit-identical."""
+@pytest.mark.parametrize("M,K,N,kernel", [(33, 128, 1, 2), (129, 384, 257, 2), (257, 4096, 33, 2), (40, 1664, 130, 2),
+                                          (260, 256, 16500, 2), (128, 896, 512, 2), (260, 128, 16300, 3),
+                                          (260, 384, 16300, 3), (260, 1280, 16300, 3), (500, 896, 16300, 3)])
+def test_int8_ring_kernel_exact(gpu, M, K, N, kernel):
+    """The prefill kernel of K % 128 == 0 with 128- (2) and 256-row (3) tiles: one
+    chunk, fewer chunks than its ring, several times as many and no multiple of
+    it, K split, part-filled rows and columns.  Sums are whole numbers below
+    2^53, exact in float64, so y must be bit-identical."""
+    from ccut._lib import lib
     from ccut.quant.int8 import int8_linear
 
+    assert lib().ccq_int8_linear_kernel(M, K, N) == kernel
     rng = np.random.default_rng(M + K + N)
     xq = rng.integers(-127, 128, (M, K)).astype(np.int8)
     w = rng.integers(-127, 128, (N, K)).astype(np.int8)

@@ -70,6 +70,17 @@ def _run(gpu, fmt, x, raw, sc, s2, N, G):
     return y.cpu().numpy()
 
 
+def _route(fmt, M, K, N, G):
+    """(kernel, rows, columns of a workgroup): 1 the 64-row kernel, 2 the 16-row
+    one, 3 the tiled one."""
+    import ctypes
+
+    from ccut._lib import lib
+
+    r, c = ctypes.c_int(), ctypes.c_int()
+    return lib().ccq_wq_linear_kernel(fmt, M, K, N, G or 32, ctypes.byref(r), ctypes.byref(c)), r.value, c.value
+
+
 FORMATS = [(FP8_ROW, 0), (INT8_ROW, 0), (MXFP8, 32), (MXFP8, 16), (MXFP4, 32), (MXFP4, 16), (MXFP4, 0)]
 
 
@@ -87,10 +98,17 @@ def test_wq_matches_oracle(gpu, fmt, G, M, K, N):
 
 
 @pytest.mark.parametrize("fmt,G", FORMATS)
-@pytest.mark.parametrize("M,K,N", [(16, 768, 4101), (3, 2304, 8190), (13, 2304, 8300), (9, 4352, 8210)])
+@pytest.mark.parametrize("M,K,N", [(5, 512, 70), (11, 1280, 4090), (16, 768, 4101), (16, 2048, 4101), (3, 2304, 8190),
+                                   (13, 2304, 8300), (13, 4096, 8300), (9, 4352, 8210), (9, 5376, 8210)])
 def test_rows_kernel_wider_blocks(gpu, fmt, G, M, K, N):
-    """Up to 16 rows on 32- and 64-column workgroups: k-tile counts that leave
-    some of the 8 waves one more than others, part-filled last columns."""
+    """Up to 16 rows on the 16-row kernel's 16-, 32- and (MXFP4) 64-column
+    workgroups, k-tile counts that leave some of the 8 waves one more than
+    others, part-filled last columns; and next to them the shapes with a short
+    K, or of 64 columns, that stay on the 64-row kernel."""
+    nb = 1 if N <= 4096 else (2 if N <= 8192 else 4)
+    stays = (nb == 2 and K == 768 and fmt != MXFP4) or (
+        nb == 4 and (fmt != MXFP4 or (G == 16 and K in (2304, 4352))))
+    assert _route(fmt, M, K, N, G) == ((1, 16, 64) if stays else (2, 16, 16 * nb))
     rng = np.random.default_rng(300 * fmt + 10 * G + M + K + N)
     raw, sc, s2, w = _case(fmt, K, N, G, rng)
     x = rng.standard_normal((M, K)).astype(np.float32)
@@ -181,13 +199,17 @@ def _apply(gpu, fmt, x, raw, sc, s2, N, G):
 
 @pytest.mark.parametrize("fmt,G", FORMATS)
 @pytest.mark.parametrize("M,K,N", [(65, 256, 8300), (129, 512, 8200), (300, 768, 4100), (13, 320, 15130),
-                                   (70, 64, 3001), (200, 1088, 1030), (270, 832, 4099)])
+                                   (70, 64, 3001), (200, 1088, 1030), (270, 832, 4099), (500, 256, 10300),
+                                   (500, 768, 10300), (260, 256, 7000), (260, 512, 7000), (260, 320, 7000),
+                                   (260, 64, 7000)])
 def test_tile_kernel_matches_oracle(gpu, fmt, G, M, K, N):
-    """The tiled kernel at each of its tile shapes (128 x 256, 128 x 128,
-    64 x 128), with part-filled rows and columns: in_features % 256 == 0 (two
+    """The tiled kernel at each of its tile shapes (128 x 256 at 500 rows, 128 x
+    128 at 260, else 64 x 128), with part-filled rows and columns: in_features % 256 == 0 (two
     activation parts, 1e-5 as above) and not (three parts, x exact: what is
     left is float32 rounding of the sums, fewer than 32 of them in a row, at
     2^-24 of a partial sum that stays within a few max|y| here)."""
+    tile = (128, 256) if M == 500 else ((128, 128) if M == 260 else (64, 128))
+    assert _route(fmt, M, K, N, G) == (3, *tile)
     rng = np.random.default_rng(7000 * fmt + 10 * G + M + K + N)
     raw, sc, s2, w = _case(fmt, K, N, G, rng)
     x = rng.standard_normal((M, K)).astype(np.float32)
