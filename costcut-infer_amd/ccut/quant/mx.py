@@ -77,8 +77,9 @@ def mx_linear(weight_bytes, scale, x, weight_dtype: str, group_size: int = 32, s
     batch, in_f = xd.shape
     raw, sc, rows = _args(weight_bytes, scale, None, in_f, fmt, group_size)
     s2 = float(1.0 if scale2 is None else np.float32(scale2))
-    # one call for every batch size: W formed in registers; from 8 rows on,
-    # in_features % 256 == 0, the products run on the matrix cores
+    # one call for every batch size: W formed in registers; the products run on
+    # the matrix cores for in_features % 256 == 0, and % 64 == 0 from about 2^17
+    # outputs on
     y = torch.empty((batch, rows), dtype=torch.float32, device=xd.device)
     call("ccq_mx_linear_f32", xd.contiguous().data_ptr(), raw.data_ptr(), sc.data_ptr() if sc is not None else None,
          y.data_ptr(), batch, in_f, rows, fmt, group_size, s2, _dev.stream_ptr())

@@ -292,7 +292,7 @@ extern "C" int ccq_mx_linear_f32(const float* x, const uint8_t* w, const uint8_t
   CCQ_REQUIRE(batch >= 0, "ccq_mx_linear_f32: negative batch");
   if (batch == 0 || out_features == 0) return 0;
   CCQ_REQUIRE(x && w && y, "ccq_mx_linear_f32: null pointer");
-  if (batch >= kMxWqMinBatch) {  // the decoded-weight MFMA kernel (-1: a shape it does not take)
+  if (batch >= kMxWqMinBatch) {  // the decoded-weight MFMA kernels (-1: a shape they do not take)
     const int rc = wq_mfma_linear(fmt == 0 ? WQ_MXFP8 : WQ_MXFP4, x, w, scale_e8m0, group_size, scale2, y, batch,
                                   in_features, out_features, as_stream(stream), "ccq_mx_linear_f32");
     if (rc >= 0) return rc;

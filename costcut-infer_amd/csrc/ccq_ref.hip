@@ -727,7 +727,7 @@ static int ref_linear(int fmt, const float* x, const uint8_t* w, const float* sc
     return launch_status(name);
   }
   // fp8 / int8 batches from kWqMinBatch* rows: the decoded-weight MFMA
-  // kernel, which reads W once per 64 rows (-1: shape it does not take)
+  // kernels (-1: shape they do not take)
   if ((fmt == 1 && batch >= kWqMinBatchFp8) || (fmt == 2 && batch >= kWqMinBatchInt8)) {
     const int rc = wq_mfma_linear(fmt == 1 ? WQ_FP8_ROW : WQ_INT8_ROW, x, w, scale, 0, 1.f, y, batch, in_f, out_f,
                                   as_stream(stream), name);

@@ -1,7 +1,7 @@
 // AWQ int4 dense GEMM above the decode kernel's 16 rows: y[M, N] = x[M, K] @ W
 // (weight and scale/zero layouts: ccq_w4.hip).
 //
-// w4_slab_kernel, 17 to 64 rows.  Everything the loop reads goes from HBM
+// w4_slab_kernel, 17 to 64 rows a workgroup.  Everything the loop reads goes from HBM
 // straight into an LDS ring (global_load_lds): activations (pieces of 16 bytes
 // XOR-swizzled by row), packed weight tiles and scale/zero words.  8 waves =
 // CG column groups x KS k-tiles of a step; a wave multiplies all 16 MT rows by

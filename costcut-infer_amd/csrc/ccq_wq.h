@@ -1,5 +1,5 @@
-// Pieces shared by the decoded-weight MFMA linears (ccq_wmfma.hip up to 64
-// rows, ccq_wtile.hip above): parameters, formats and the in-register decode.
+// Pieces shared by the decoded-weight MFMA linears (ccq_wrows.hip up to 16 rows,
+// ccq_wmfma.hip up to 64 rows a workgroup, ccq_wtile.hip above): parameters, formats and the in-register decode.
 #pragma once
 
 #include "ccq_common.h"
